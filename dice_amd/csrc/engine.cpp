@@ -222,8 +222,8 @@ void Engine::loadSystem(HostSystem&& sys) {
   if (storage && std::strcmp(storage, "half") == 0) storageMode = 1;
   if (storage && std::strcmp(storage, "full") == 0) storageMode = -1;
   // SHCI_HALF_SIGMA=rows: half storage's sigma on the stored rows (no tiled
-  // copy); SHCI_HALF_STAGE_MIN=k: segments of at least k instructions sum
-  // their transposed products in LDS first (1: every segment)
+  // copy); SHCI_HALF_STAGE_MIN=k: a tile with at least k instructions in 1,024
+  // rows has its x and transposed sums in LDS (1: every tile)
   if (const char* p = std::getenv("SHCI_HALF_SIGMA")) lowerTiled = std::strcmp(p, "rows") != 0;
   if (const char* p = std::getenv("SHCI_HALF_STAGE_MIN")) lowerStageMin = std::max(1, std::atoi(p));
   // SHCI_HALF_SPLIT=1: split columns in the half's tiled copy too
@@ -819,8 +819,7 @@ void Engine::buildLower(int64_t nOld) {
   if (std::getenv("SHCI_TIMING"))
     std::fprintf(stderr, "# half-storage build n=%lld: %lld stored off-diagonal elements\n", (long long)n,
                  (long long)total);
-  const int64_t nnzOld = nOld ? nnzOff : 0;
-  const int64_t added = total - nnzOld;
+  const int64_t added = total - (nOld ? nnzOff : 0);
   {
     size_t totalB = 0;
     const size_t freeB = deviceFreeBytes(&totalB);
@@ -847,15 +846,14 @@ void Engine::buildLower(int64_t nOld) {
   nnzOff = total;
   hamRows = n;
   permRows = -1;
-  buildLowerTiled(nOld, nnzOld);
+  buildLowerTiled();
   HIP_CHECK(hipStreamSynchronize(stream));
 }
 
 // The tiled copy of the stored half, built from it through the alpha-major
 // relabelling (and the split columns when their x copy fits), when it fits
-// beside it with the permuted x and the transposed sums (nOld, nnzOld: the
-// rows and entries kept from the previous build).
-void Engine::buildLowerTiled(int64_t nOld, int64_t nnzOld) {
+// beside it with the permuted x and the sums.
+void Engine::buildLowerTiled() {
   tiledRows = -1;
   splitRows = -1;
   if (!relabel || !tiledOn || !lowerTiled || n == 0) return;
@@ -879,24 +877,15 @@ void Engine::buildLowerTiled(int64_t nOld, int64_t nnzOld) {
   if (!buildTiledHam(tiled, rowPtr.as<int64_t>(), cols.as<int32_t>(), f32 ? nullptr : vals.as<double>(),
                      f32 ? vals32.as<float>() : nullptr, perm, permPos.as<uint32_t>(),
                      doSplit ? T.bIdx.as<uint32_t>() : nullptr, doSplit ? bPos.as<uint32_t>() : nullptr, n, nnzOff,
-                     ws, stream, false, lowerStageMin, f32 ? valsLo.as<float>() : nullptr)) {
+                     ws, stream, false, lowerStageMin, f32 ? valsLo.as<float>() : nullptr, true)) {
     tiled.release();
     return;
   }
   const int64_t nx = doSplit ? 2 * n : n;
   lowerYT.reserve((size_t)(nx + 1) * 8);
-  // the row sums grow with the half: when they cover exactly the rows kept
-  // from the previous build, only the added rows are summed
-  const bool grow = nOld > 0 && lowerAbsRows == nOld && lowerAbsNnz == nnzOld && lowerAbsF32 == f32;
-  const int64_t r0 = grow ? lowerAbsRows : 0;
-  lowerRowAbs.reserve((size_t)n * 8, stream, grow);
   lowerBound.reserve(8);
-  launchSymRowBound(rowPtr.as<int64_t>(), cols.as<int32_t>(), f32 ? nullptr : vals.as<double>(),
-                    f32 ? vals32.as<float>() : nullptr, r0, n, lowerRowAbs.as<unsigned long long>(),
-                    lowerBound.as<unsigned long long>(), stream);
-  lowerAbsRows = n;
-  lowerAbsNnz = nnzOff;
-  lowerAbsF32 = f32;
+  launchSymRowBound(tiled, permPos.as<uint32_t>(), doSplit ? bPos.as<uint32_t>() : nullptr,
+                    lowerYT.as<unsigned long long>(), lowerBound.as<unsigned long long>(), stream);
   tiledRows = n;
   if (doSplit) splitRows = n;
 }

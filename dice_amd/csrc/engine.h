@@ -101,21 +101,16 @@ struct Engine {
   // gathered in lowerYT (fixed point, permuted order; then max|x|); the FP32
   // form's exact sigma keeps the row kernel
   bool lowerTiled = true;
-  // instructions that make a segment large (sigma on the 24-orbital
-  // workload, 1: 3.42, 2: 3.22, 3: 3.10, 4: 3.09, 6: 3.28, 8: 3.59 ms; 16
-  // instructions per wave per step instead of 8: 12% slower)
-  int lowerStageMin = 4;
+  // instructions of one tile in a super block that make its group large (sigma
+  // on 1,000,003 determinants of 24 orbitals, 4: 1,895, 6: 1,716, 8: 1,701,
+  // 12: 1,918 us; on 200,003: 314, 247, 239, 265)
+  int lowerStageMin = 8;
   // split columns in the half's tiled copy (sigma on the 24-orbital
   // workload: 3.08 ms with, 2.96 ms without, and a shorter build)
   bool lowerSplit = false;
   DevMem lowerYT;
-  // the off-diagonal row sums of |H| (fixed point) over the first
-  // lowerAbsRows rows' stored entries, grown with the half, and their
-  // largest (kSigmaTiledSym's bound)
-  DevMem lowerRowAbs, lowerBound;
-  int64_t lowerAbsRows = -1, lowerAbsNnz = 0;
-  bool lowerAbsF32 = false;
-  void buildLowerTiled(int64_t nOld, int64_t nnzOld);
+  DevMem lowerBound;  // the largest off-diagonal row sum of |H| (kSigmaTiledSym's scale)
+  void buildLowerTiled();
 
   // Davidson scratch
   DevMem dvB, dvS, dvR, dvScal, dvPart, dvG, dvW, dvV, dvX;

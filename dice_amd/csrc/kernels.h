@@ -262,6 +262,10 @@ struct TiledHam {
   bool f32 = false, split = false, hasLo = false;
   // lo: the FP32 values' remainders (lo = fp32(v - hi)), when built with them
   DevMem segBase, segTile, segCnt, segStart, segInst, segTotal, fill, blockE, blockI, idx, vals, lo, inst;
+  // the half-storage sigma's order: the segments by (super block, tile, row
+  // block), its instructions (symInst), tile groups and work units
+  DevMem order, blockOf, bigI, smallI, lead, groups, symInst, unitStart, units;
+  int64_t unitCap = 0;
   void release();
 };
 // device bytes buildTiledHam needs for nnz entries over n rows (upper bound
@@ -275,14 +279,15 @@ size_t tiledHamBytes(int64_t n, int64_t nnz, bool f32);
 // itself (rows and columns already permuted; splitCols says whether its
 // columns reach into the beta-major copy).  Segments of at least stageMin
 // instructions are marked as large (the staged sigma copies their x tile to
-// LDS; the half-storage sigma sums their transposed products there).  With
-// vals32, valsLo (the FP32 remainders) is copied beside them when given.
+// LDS).  With vals32, valsLo (the FP32 remainders) is copied beside them when
+// given.  sym: for the half-storage sigma, whose order of the copy is built
+// too, with groups of at least stageMin instructions as large ones.
 // Returns false, with nothing built, when the permuted x has more tiles than
 // the build's bitmap holds.
 bool buildTiledHam(TiledHam& T, const int64_t* rowPtr, const int32_t* cols, const double* vals64,
                    const float* vals32, const uint32_t* perm, const uint32_t* pos, const uint32_t* bIdx,
                    const uint32_t* bPos, int64_t n, int64_t nnz, Workspace& ws, hipStream_t s,
-                   bool splitCols = false, int stageMin = 8, const float* valsLo = nullptr);
+                   bool splitCols = false, int stageMin = 8, const float* valsLo = nullptr, bool sym = false);
 // y = H x through the tiled copy (one vector, x and y in determinant order;
 // bPerm = the beta-major determinant order when the copy has split columns)
 // (step: instructions per wave per step, 8 or 16; stage: each wave copies
@@ -301,12 +306,10 @@ void launchSigmaTiledSym(const TiledHam& T, const double* diag, const uint32_t* 
                          const uint32_t* pos, const uint32_t* bPos, const double* x, double* y, const XScratch& xP,
                          unsigned long long* yT, const unsigned long long* bound, hipStream_t s, bool exact = false);
 // kSigmaTiledSym's bound (the largest off-diagonal row sum of |H|) into
-// *bound, from the row sums in acc (n words): the rows [nOld, n) of a half
-// grown from nOld rows (CSR rowPtr, cols, values: vals64 or vals32, as
-// stored) are added to the sums of the first nOld rows (nOld = 0 for a new
-// half).
-void launchSymRowBound(const int64_t* rowPtr, const int32_t* cols, const double* vals64, const float* vals32,
-                       int64_t nOld, int64_t n, unsigned long long* acc, unsigned long long* bound, hipStream_t s);
+// *bound, from the tiled copy itself; pos / bPos as above, yT: nx words of
+// scratch.
+void launchSymRowBound(const TiledHam& T, const uint32_t* pos, const uint32_t* bPos, unsigned long long* yT,
+                       unsigned long long* bound, hipStream_t s);
 
 // --- Davidson vector kernels ----------------------------------------------------------
 // G[i*mb + j] = A[:,i] . B[:,j] for i < ma, j < mb (columns of length n, ld)

@@ -1755,7 +1755,7 @@ __global__ void __launch_bounds__(kBlock) kSigmaLower(const int64_t* __restrict_
 // the entries are ordered by the wave that placed them (row mod 4), then by
 // row, then in the row's own order, so each row is one contiguous run; an
 // instruction's products are summed per row by a segmented scan across
-// lanes (each entry carries its distance to its run's first entry) and
+// lanes (each entry carries which of its steps add to it) and
 // added into the executing wave's partial row sums in LDS, and the four
 // partials are added in a fixed order at the end of the block.  Which wave
 // takes which instructions is fixed by the layout, so the result does not
@@ -1767,10 +1767,11 @@ constexpr int kTileCols = 1 << kTileLog;
 constexpr int kTileMaxWords = 4096;  // bitmap of up to 131,072 tiles: x of up to 134M values
 constexpr int kTileInstPad = 16;  // zero descriptors after the last one (the largest step of kSigmaTiled)
 constexpr int kTileLdsSegs = 1024;  // blocks with at most this many segments count and fill in LDS
-// an entry's 32-bit word: column in tile (bits 0-9), distance to the first
-// entry of its row run within the instruction (bits 10-15), row in block
-// (bits 16-23), last entry of its run within the instruction (bit 31)
-constexpr int kTileDistShift = 10;
+// an entry's 32-bit word: column in tile (bits 0-9), which of the six steps
+// of the segmented scan of its instruction add to it (bits 10-15,
+// segInclusiveScan), row in block (bits 16-23), last entry of its row run
+// within the instruction (bit 31)
+constexpr int kTileStepShift = 10;
 // an instruction descriptor: its first entry (offset within the block),
 // and a second word with the entry count (bits 0-6), the tile (bits 7-30),
 // and bit 31 set when its segment has at least stageMin
@@ -2016,9 +2017,27 @@ __global__ void __launch_bounds__(kBlock) kTileFill(const int64_t* rowPtr, const
   }
 }
 
-// pass 4: per entry, its distance to the first entry of its row run within
-// its instruction and whether it is the run's last entry there (one wave
-// per instruction)
+// The scan of an instruction's products: a segmented inclusive scan across
+// the wave by DPP, whose steps are row_shr 1, 2, 4, 8 (within rows of 16
+// lanes), row_bcast 15 (lane 15 into row 1, lane 47 into row 3) and row_bcast
+// 31 (lane 31 into rows 2 and 3).  A lane adds a step's value when the lane it
+// comes from lies in its run: by its distance `dist` to its run's first lane,
+// counted within its row for the shifts.  Runs are contiguous, so every lane
+// ends with the sum of its run up to itself.
+__device__ __forceinline__ uint32_t segScanSteps(int lane, int dist) {
+  const int col = lane & 15, inRow = dist < col ? dist : col;
+  uint32_t m = 0;
+  m |= inRow >= 1 ? 1u : 0u;
+  m |= inRow >= 2 ? 2u : 0u;
+  m |= inRow >= 4 ? 4u : 0u;
+  m |= inRow >= 8 ? 8u : 0u;
+  m |= ((lane >> 4) & 1) && dist > col ? 16u : 0u;
+  m |= lane >= 32 && dist >= lane - 31 ? 32u : 0u;
+  return m;
+}
+
+// pass 4: per entry, the scan steps that add to it and whether it is the last
+// of its row run within its instruction (one wave per instruction)
 __global__ void __launch_bounds__(kBlock) kTileRunBits(const uint2* __restrict__ inst,
                                                        const int64_t* __restrict__ blockI,
                                                        const int64_t* __restrict__ blockE, uint32_t* tIdx) {
@@ -2039,49 +2058,31 @@ __global__ void __launch_bounds__(kBlock) kTileRunBits(const uint2* __restrict__
     // the highest run start at or below this lane
     const unsigned long long upTo = starts & (~0ull >> (63 - lane));
     const int first = 63 - __clzll(upTo);
-    const uint32_t dist = (uint32_t)(lane - first);
     if (valid)
-      tIdx[p] = (ix & ~((63u << kTileDistShift) | 0x80000000u)) | (dist << kTileDistShift) | (last ? 0x80000000u : 0u);
+      tIdx[p] = (ix & ~((63u << kTileStepShift) | 0x80000000u)) | (segScanSteps(lane, lane - first) << kTileStepShift) |
+                (last ? 0x80000000u : 0u);
   }
 }
 
-// One step of a segmented inclusive scan across the wave by DPP: lane i
-// adds the value of the lane the DPP control CTRL names (within the rows of
-// 16 lanes ROWMASK enables) when that lane lies in its run, i.e. when the
-// lane's distance to the first lane of its run is at least `need` (need is
-// larger than any distance where CTRL brings no value into the lane, so the
-// value a disabled or out-of-row lane receives is never used).  Runs are
-// contiguous, so the steps row_shr 1, 2, 4, 8 (distance counted within the
-// row of 16), then row_bcast 15 and row_bcast 31 give every lane the sum of
-// its run up to itself.
-template <int CTRL, int ROWMASK>
-__device__ __forceinline__ void segScanStep(double& s, int dist, int need) {
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(s), CTRL, ROWMASK, 0xf, false);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(s), CTRL, ROWMASK, 0xf, false);
-  if (dist >= need) s += __hiloint2double(hi, lo);
+// One step: the value DPP control CTRL brings, masked to zero where the
+// entry word's step bit is not set (an AND that takes the DPP operand itself;
+// adding zero changes no bit of a sum but the sign of a zero).
+template <int CTRL>
+__device__ __forceinline__ void segScanStep(double& s, uint32_t ix, int bit) {
+  const int m = (int)(ix << (31 - kTileStepShift - bit)) >> 31;
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(s), CTRL, 0xf, 0xf, true) & m;
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(s), CTRL, 0xf, 0xf, true) & m;
+  s += __hiloint2double(hi, lo);
 }
 
-// dist: the lane's distance to the first lane of its run (runs contiguous);
-// c15, c31: per-lane thresholds of the two broadcast steps (tileScanConsts)
-__device__ __forceinline__ double segInclusiveScan(double s, int dist, int c15, int c31) {
-  const int inRow = dist < (int)(__lane_id() & 15u) ? dist : (int)(__lane_id() & 15u);
-  segScanStep<0x111, 0xf>(s, inRow, 1);  // row_shr:1
-  segScanStep<0x112, 0xf>(s, inRow, 2);  // row_shr:2
-  segScanStep<0x114, 0xf>(s, inRow, 4);  // row_shr:4
-  segScanStep<0x118, 0xf>(s, inRow, 8);  // row_shr:8
-  segScanStep<0x142, 0xa>(s, dist, c15);  // row_bcast:15 (lane 15 into row 1, lane 47 into row 3)
-  segScanStep<0x143, 0xc>(s, dist, c31);  // row_bcast:31 (lane 31 into rows 2 and 3)
+__device__ __forceinline__ double segInclusiveScan(double s, uint32_t ix) {
+  segScanStep<0x111>(s, ix, 0);  // row_shr:1
+  segScanStep<0x112>(s, ix, 1);  // row_shr:2
+  segScanStep<0x114>(s, ix, 2);  // row_shr:4
+  segScanStep<0x118>(s, ix, 3);  // row_shr:8
+  segScanStep<0x142>(s, ix, 4);  // row_bcast:15
+  segScanStep<0x143>(s, ix, 5);  // row_bcast:31
   return s;
-}
-
-// the broadcast steps' thresholds: a lane of row 1 or 3 takes the previous
-// row's last lane when that lane is in its run (distance > its index in the
-// row); a lane of row 2 or 3 takes lane 31 when the distance reaches back to
-// it; other lanes never take the broadcast value
-__device__ __forceinline__ void tileScanConsts(int& c15, int& c31) {
-  const int lane = (int)__lane_id();
-  c15 = ((lane >> 4) & 1) ? (lane & 15) + 1 : 64;
-  c31 = lane >= 32 ? lane - 31 : 64;
 }
 
 // y[perm[m]] = diag .* x + (H x) over the tiled copy, one vector; xP holds x
@@ -2125,8 +2126,6 @@ __global__ void __launch_bounds__(kBlock) kSigmaTiled(const uint2* __restrict__ 
   __shared__ __align__(16) XT xs[STAGE ? kWaves : 1][STAGE ? kTileCols : 1];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = __lane_id();
   static_assert(U <= kTileInstPad, "step larger than the descriptor padding");
-  int c15, c31;
-  tileScanConsts(c15, c31);
   uint32_t staged = 0xffffffffu;  // the tile in this wave's LDS (x does not change within a launch)
   ChunkSched<1, PERSIST> sched{nblocks, counter, -1};
   while (sched.next()) {
@@ -2197,7 +2196,7 @@ __global__ void __launch_bounds__(kBlock) kSigmaTiled(const uint2* __restrict__ 
 #pragma unroll
       for (int u = 0; u < U; u++) {
         const bool valid = (uint32_t)lane < (dy[u] & 127u);
-        const double sum = segInclusiveScan(v[u] * xv[u], (int)((ix[u] >> kTileDistShift) & 63u), c15, c31);
+        const double sum = segInclusiveScan(v[u] * xv[u], ix[u]);
         if (valid && (int)ix[u] < 0) yw[wave][(ix[u] >> 16) & (kTileRows - 1)] += sum;
       }
     }
@@ -2224,108 +2223,277 @@ __global__ void __launch_bounds__(kBlock) kSigmaTiled(const uint2* __restrict__ 
 // row sum of |H_IJ|), so no row's sum of integers reaches 2^62 in
 // magnitude, and each integer is off by at most 2^(e-1) (below
 // 2^-61 B max|x|).  Row parts: each instruction's products are summed per
-// row run in FP64 by the segmented scan, and each run's sum is added as an
-// integer into the block's row sums in LDS, which go to yT at the end.
-// Transposed parts: each wave sums its current tile's integers in LDS
-// (segments with the large-segment bit; the others add theirs into yT
-// directly) and adds the nonzero sums into yT with 64-bit integer atomics
-// when its tile changes.  Each wave takes a contiguous quarter of its
-// block's instructions.  yT: nx sums (cleared first), then the bits of
-// max|x|; bound: the bits of B.
-__device__ __forceinline__ int symFixExp(const unsigned long long* yT, int64_t nx, const unsigned long long* bound) {
-  const double S = __longlong_as_double((long long)yT[nx]) * __longlong_as_double((long long)*bound);
-  return S > 0.0 && S <= DBL_MAX ? ilogb(S) + 1 - 61 : 0;  // (x holding inf: no scale is right)
+// row run in FP64 by the segmented scan, and each run's sum is one integer.
+// Transposed parts: every product is one.  yT: nx sums (cleared first), then
+// the bits of max|x|; bound: the bits of B.
+//
+// How the work is cut changes no bit, so the instructions are taken in an
+// order of their own: kSymBlocks row blocks form a super block, whose
+// instructions are sorted by tile (SymOrder).  A workgroup then keeps the x
+// and the sums of the super block's rows and of the current tile's columns
+// in LDS (32 KB, four workgroups of 512 threads per CU) for all the entries
+// of that tile, so that nothing but the entries is read from memory per
+// entry, and a tile's sums are added to yT once for 1,024 rows.  Bound by the
+// scan's VALU work and the LDS adds beside HBM.
+//
+// Measured, one product, against a workgroup per row block whose four waves
+// each kept a tile's transposed sums of their own and gathered x through L1:
+// 2,471 determinants of 16 orbitals 61 -> 15 us, 27,685 of 24 orbitals 423 ->
+// 55, 57,963 of 40 orbitals 371 -> 89, 200,003 of 24 orbitals 569 -> 239,
+// 1,000,003 of them (4.7e8 pairs) 2,569 -> 1,700 (3.3 TB/s over 12 bytes a
+// pair), 300,007 of 40 orbitals with FP32 values 1,930 -> 980.  Super blocks
+// of 2 and 8 blocks: 2,000 and 1,700 us on the million, 97 and 90 on the
+// 57,963; 256 threads: 1,990 and 109; 2 and 8 instructions at a time: 1,730
+// and 1,800.
+constexpr int kSymBlocks = 4;
+constexpr int kSymRows = kSymBlocks * kTileRows;
+constexpr int kSymThreads = 512;
+constexpr int kSymWaves = kSymThreads / 64;
+constexpr int kSymStep = 4;  // instructions a wave loads together
+// an instruction's second word in this order: entries (bits 0-6), row block in
+// its super block (7-9), tile (10-31)
+constexpr int kSymTileShift = 10;
+constexpr uint32_t kSymSmall = 0x80000000u;
+
+// a workgroup's work: `len` instructions of super block `sb` from `first` on,
+// which lies in tile group `group`; with kSymSmall in sb, instructions of
+// small groups.  len 0: unused.
+struct __align__(16) SymUnit {
+  uint32_t sb, first, len, group;
+};
+
+// place of every segment in the order (super block, tile, row block); per
+// place its instructions as one of a large group (the instructions of one
+// tile in one super block, at least bigMin) or of a small one, and whether
+// it begins a large group
+__global__ void kSymRank(const int64_t* __restrict__ segBase, int64_t blocks, int64_t segs,
+                         const uint32_t* __restrict__ segTile, const uint32_t* __restrict__ segTotal, uint32_t bigMin,
+                         uint32_t* order, uint32_t* blockOf, int64_t* bigI, int64_t* smallI, int64_t* lead) {
+  for (int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; s < segs; s += (int64_t)gridDim.x * blockDim.x) {
+    int64_t lo = 0, hi = blocks - 1;  // the last block that begins at or before s
+    while (lo < hi) {
+      const int64_t mid = (lo + hi + 1) >> 1;
+      if (segBase[mid] <= s)
+        lo = mid;
+      else
+        hi = mid - 1;
+    }
+    const int64_t b = lo, q0 = b / kSymBlocks * kSymBlocks;
+    const int64_t q1 = q0 + kSymBlocks < blocks ? q0 + kSymBlocks : blocks;
+    const uint32_t tile = segTile[s];
+    int64_t at = segBase[q0];
+    uint32_t total = 0;
+    bool first = true;
+    for (int64_t c = q0; c < q1; c++) {
+      int64_t i = segBase[c], j = segBase[c + 1];
+      const int64_t c0 = i, c1 = j;
+      while (i < j) {  // block c's first segment with a tile >= this one's
+        const int64_t mid = (i + j) >> 1;
+        if (segTile[mid] < tile)
+          i = mid + 1;
+        else
+          j = mid;
+      }
+      at += i - c0;
+      if (i < c1 && segTile[i] == tile) {
+        total += (segTotal[i] + 63u) / 64u;
+        if (c < b) {
+          at++;
+          first = false;
+        }
+      }
+    }
+    const int64_t mine = (segTotal[s] + 63u) / 64u;
+    const bool big = total >= bigMin;
+    order[at] = (uint32_t)s;
+    blockOf[at] = (uint32_t)b;
+    bigI[at] = big ? mine : 0;
+    smallI[at] = big ? 0 : mine;
+    lead[at] = big && first ? 1 : 0;
+  }
 }
 
-template <typename VT, typename XT, int U, bool LO>
-__global__ void __launch_bounds__(kBlock) kSigmaTiledSym(const uint2* __restrict__ inst,
-                                                         const int64_t* __restrict__ blockI,
-                                                         const int64_t* __restrict__ blockE,
-                                                         const uint32_t* __restrict__ tIdx,
-                                                         const VT* __restrict__ tVal,
-                                                         const float* __restrict__ tLo, int64_t n, int64_t nx,
-                                                         const XT* __restrict__ xP, unsigned long long* yT,
-                                                         const unsigned long long* __restrict__ bound) {
-  __shared__ unsigned long long yr[kTileRows];          // the block's row sums
-  __shared__ unsigned long long ya[kWaves][kTileCols];  // the wave's current tile of transposed sums
-  __shared__ double xr[kTileRows];                      // x of the block's rows, times 2^-e
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = __lane_id();
-  static_assert(U <= kTileInstPad, "step larger than the descriptor padding");
-  int c15, c31;
-  tileScanConsts(c15, c31);
-  const int e = symFixExp(yT, nx, bound);
-  const int64_t b = blockIdx.x;
-  const int64_t m0 = b * kTileRows;
-  for (int j = lane; j < kTileCols; j += 64) ya[wave][j] = 0ull;
-  for (int t = threadIdx.x; t < kTileRows; t += kBlock) {
-    yr[t] = 0ull;
-    xr[t] = m0 + t < n ? ldexp((double)xP[m0 + t], -e) : 0.0;
+// the instructions in that order, those of large groups first, and the large
+// groups (bigI, smallI, lead: scanned)
+__global__ void kSymEmit(int64_t segs, const uint32_t* __restrict__ order, const uint32_t* __restrict__ blockOf,
+                         const int64_t* __restrict__ blockE, const uint32_t* __restrict__ segTile,
+                         const uint32_t* __restrict__ segTotal, const uint32_t* __restrict__ segStart,
+                         const int64_t* __restrict__ bigI, const int64_t* __restrict__ smallI,
+                         const int64_t* __restrict__ lead, uint2* inst, uint2* groups) {
+  const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t nBig = bigI[segs];
+  for (int64_t p = tid; p < segs; p += (int64_t)gridDim.x * blockDim.x) {
+    const uint32_t s = order[p], b = blockOf[p], tile = segTile[s], total = segTotal[s];
+    const uint32_t rel = (uint32_t)(blockE[b] - blockE[b / kSymBlocks * kSymBlocks]) + segStart[s];
+    const bool big = bigI[p + 1] != bigI[p];
+    const int64_t at = big ? bigI[p] : nBig + smallI[p];
+    for (uint32_t j = 0; 64u * j < total; j++)
+      inst[at + j] = make_uint2(rel + 64u * j, (total - 64u * j < 64u ? total - 64u * j : 64u) |
+                                                   ((b % kSymBlocks) << 7) | (tile << kSymTileShift));
+    if (lead[p + 1] != lead[p]) groups[lead[p]] = make_uint2((uint32_t)bigI[p], tile);
   }
-  __syncthreads();
-  uint32_t cur = 0xffffffffu;
-  auto flush = [&](uint32_t tile) {
-    for (int j = lane; j < kTileCols; j += 64) {
-      const unsigned long long a = ya[wave][j];
-      if (a != 0ull) {
-        atomicAdd(&yT[((size_t)tile << kTileLog) + j], a);
-        ya[wave][j] = 0ull;
+  if (tid == 0) groups[lead[segs]] = make_uint2((uint32_t)nBig, 0u);
+}
+
+// units per super block (units null), or the units themselves from the
+// scanned counts; those past the last are marked unused
+__global__ void kSymUnits(const int64_t* __restrict__ segBase, int64_t blocks, int64_t supers, int64_t segs,
+                          const int64_t* __restrict__ bigI, const int64_t* __restrict__ smallI,
+                          const int64_t* __restrict__ lead, const uint2* __restrict__ groups, int64_t per,
+                          int64_t* unitStart, SymUnit* units, int64_t cap) {
+  const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t q = tid; q < supers; q += step) {
+    const int64_t p0 = segBase[q * kSymBlocks];
+    const int64_t p1 = segBase[(q + 1) * kSymBlocks < blocks ? (q + 1) * kSymBlocks : blocks];
+    const int64_t b0 = bigI[p0], b1 = bigI[p1], s0 = bigI[segs] + smallI[p0], s1 = bigI[segs] + smallI[p1];
+    if (!units) {
+      unitStart[q] = (b1 - b0 + per - 1) / per + (s1 - s0 + per - 1) / per;
+      continue;
+    }
+    SymUnit* u = units + unitStart[q];
+    for (int64_t i = b0; i < b1; i += per) {
+      int64_t a = lead[p0], b = lead[p1] - 1;  // the last group that begins at or before i
+      while (a < b) {
+        const int64_t mid = (a + b + 1) >> 1;
+        if ((int64_t)groups[mid].x <= i)
+          a = mid;
+        else
+          b = mid - 1;
+      }
+      *u++ = SymUnit{(uint32_t)q, (uint32_t)i, (uint32_t)(b1 - i < per ? b1 - i : per), (uint32_t)a};
+    }
+    for (int64_t i = s0; i < s1; i += per)
+      *u++ = SymUnit{(uint32_t)q | kSymSmall, (uint32_t)i, (uint32_t)(s1 - i < per ? s1 - i : per), 0u};
+  }
+  if (!units) {
+    if (tid == 0) unitStart[supers] = 0;
+    return;
+  }
+  for (int64_t u = unitStart[supers] + tid; u < cap; u += step) units[u] = SymUnit{0u, 0u, 0u, 0u};
+}
+
+__device__ __forceinline__ double symFixRange(const unsigned long long* yT, int64_t nx,
+                                              const unsigned long long* bound) {
+  return __longlong_as_double((long long)yT[nx]) * __longlong_as_double((long long)*bound);
+}
+__device__ __forceinline__ int symFixExp(double range) {
+  return range > 0.0 && range <= DBL_MAX ? ilogb(range) + 1 - 61 : 0;
+}
+
+// the integer nearest t (ties to even), |t| < 2^62, from four additions: t
+// rounded to a multiple of 2^32 has that multiple in the low mantissa bits of
+// t + 1.5 2^84, and the rest, exact and at most 2^31, its nearest integer in
+// those of rest + 1.5 2^52.  (__double2ll_rn takes seven operations, most of
+// them at a lower rate.)
+__device__ __forceinline__ unsigned long long fixRound(double t) {
+  const double a = t + 0x1.8p84;
+  const double rest = t - (a - 0x1.8p84);
+  const uint32_t hi = (uint32_t)__double2loint(a);
+  const double b = rest + 0x1.8p52;
+  return ((unsigned long long)((uint32_t)__double2hiint(b) - 0x43380000u + hi) << 32) | (uint32_t)__double2loint(b);
+}
+
+// ABS: the row sums of |H| for the bound B, every |v| rounded up to a multiple
+// of 2^-32 and summed as an integer (x is not read)
+template <typename VT, typename XT, bool LO, bool ABS>
+__global__ void __launch_bounds__(kSymThreads) kSigmaTiledSym(const SymUnit* __restrict__ units,
+                                                              const uint2* __restrict__ inst,
+                                                              const uint2* __restrict__ groups,
+                                                              const int64_t* __restrict__ blockE,
+                                                              const uint32_t* __restrict__ tIdx,
+                                                              const VT* __restrict__ tVal,
+                                                              const float* __restrict__ tLo, int64_t n, int64_t nx,
+                                                              const XT* __restrict__ xP, unsigned long long* yT,
+                                                              const unsigned long long* __restrict__ bound) {
+  __shared__ unsigned long long yr[kSymRows], yc[kTileCols];
+  __shared__ double xr[kSymRows], xc[kTileCols];  // xr: times 2^-e
+  const SymUnit unit = units[blockIdx.x];
+  if (unit.len == 0u) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = __lane_id();
+  const int e = ABS ? 0 : symFixExp(symFixRange(yT, nx, bound));
+  const bool small = (unit.sb & kSymSmall) != 0u;
+  const int64_t sb = unit.sb & ~kSymSmall, m0 = sb * kSymRows, e0 = blockE[sb * kSymBlocks];
+  for (int j = threadIdx.x; j < kSymRows; j += kSymThreads) {
+    yr[j] = 0ull;
+    xr[j] = !ABS && m0 + j < n ? ldexp((double)xP[m0 + j], -e) : 0.0;
+  }
+  for (int j = threadIdx.x; j < kTileCols; j += kSymThreads) yc[j] = 0ull;
+  // instructions [a, b) of one tile (staged) or of any (x and transposed sums
+  // in memory), by one wave
+  auto run = [&](uint32_t a, uint32_t b, bool staged) {
+    for (uint32_t i = a; i < b; i += kSymStep) {
+      uint32_t dx[kSymStep], dy[kSymStep], ix[kSymStep];
+      double v[kSymStep];
+#pragma unroll
+      for (int u = 0; u < kSymStep; u++) {
+        const uint2 d = inst[i + u < b ? i + u : a];
+        dx[u] = d.x;
+        dy[u] = i + u < b ? d.y : (d.y & ~127u);  // no entries past the range
+      }
+#pragma unroll
+      for (int u = 0; u < kSymStep; u++) {
+        ix[u] = 0u;
+        v[u] = 0.0;
+        if ((uint32_t)lane < (dy[u] & 127u)) {
+          const int64_t p = e0 + dx[u] + lane;
+          ix[u] = __builtin_nontemporal_load(tIdx + p);
+          v[u] = (double)__builtin_nontemporal_load(tVal + p);
+          if (LO) v[u] += (double)__builtin_nontemporal_load(tLo + p);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kSymStep; u++) {
+        const uint32_t cnt = dy[u] & 127u;
+        if (cnt == 0u) continue;
+        const bool valid = (uint32_t)lane < cnt;
+        const uint32_t row = ((ix[u] >> 16) & (kTileRows - 1)) + (((dy[u] >> 7) & 7u) * kTileRows);
+        const uint32_t col = ix[u] & (uint32_t)(kTileCols - 1);
+        const size_t k0 = (size_t)(dy[u] >> kSymTileShift) << kTileLog;
+        unsigned long long q;
+        if (ABS) {
+          q = (unsigned long long)ceil(ldexp(fabs(v[u]), 32));
+          if (valid) atomicAdd(&yr[row], q);
+        } else {
+          const double xv = staged ? xc[col] : (double)xP[k0 + col];
+          const double sum = segInclusiveScan(v[u] * xv, ix[u]);
+          if (valid && (int)ix[u] < 0) atomicAdd(&yr[row], fixRound(ldexp(sum, -e)));
+          q = fixRound(v[u] * xr[row]);
+        }
+        if (staged) {
+          if (valid) atomicAdd(&yc[col], q);
+        } else if (valid && q != 0ull) {
+          atomicAdd(&yT[k0 + col], q);
+        }
       }
     }
   };
-  const int64_t i0 = blockI[b], i1 = blockI[b + 1], e0 = blockE[b];
-  const int64_t len = i1 - i0;
-  const int64_t w0 = i0 + len * wave / kWaves, wEnd = i0 + len * (wave + 1) / kWaves;
-  for (int64_t i = w0; i < wEnd; i += U) {
-    uint32_t dx[U], dy[U];
-    const uint2* dp = inst + i;
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const uint2 d = dp[u];
-      dx[u] = d.x;
-      dy[u] = i + u < wEnd ? d.y : (d.y & ~127u);  // count 0 past the range
-    }
-    uint32_t ix[U];
-    double v[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const bool valid = (uint32_t)lane < (dy[u] & 127u);
-      const int64_t p = e0 + (valid ? (int64_t)dx[u] + lane : 0);
-      ix[u] = __builtin_nontemporal_load(tIdx + p);
-      v[u] = (double)__builtin_nontemporal_load(tVal + p);
-      if (LO) v[u] += (double)__builtin_nontemporal_load(tLo + p);
-    }
-    double xv[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const bool valid = (uint32_t)lane < (dy[u] & 127u);
-      const size_t tb = (size_t)((dy[u] >> 7) & kTileDescMask) << kTileLog;
-      xv[u] = (double)xP[tb + (valid ? (ix[u] & (uint32_t)(kTileCols - 1)) : 0u)];
-    }
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      if ((dy[u] & 127u) == 0) continue;
-      const bool valid = (uint32_t)lane < (dy[u] & 127u);
-      const uint32_t row = (ix[u] >> 16) & (kTileRows - 1);
-      const double sum = segInclusiveScan(v[u] * xv[u], (int)((ix[u] >> kTileDistShift) & 63u), c15, c31);
-      if (valid && (int)ix[u] < 0) atomicAdd(&yr[row], (unsigned long long)__double2ll_rn(ldexp(sum, -e)));
-      const uint32_t tile = (dy[u] >> 7) & kTileDescMask;
-      const uint32_t col = ix[u] & (uint32_t)(kTileCols - 1);
-      const unsigned long long q = (unsigned long long)__double2ll_rn(v[u] * xr[row]);
-      if (!(dy[u] >> 31)) {
-        if (valid && q != 0ull) atomicAdd(&yT[((size_t)tile << kTileLog) + col], q);
-        continue;
+  const uint32_t end = unit.first + unit.len;
+  if (small) {
+    __syncthreads();
+    run(unit.first + unit.len * wave / kSymWaves, unit.first + unit.len * (wave + 1) / kSymWaves, false);
+  } else {
+    uint32_t at = unit.first;
+    for (uint32_t g = unit.group; at < end; g++) {
+      const uint32_t tile = groups[g].y, next = groups[g + 1].x, to = next < end ? next : end, len = to - at;
+      const int64_t k0 = (int64_t)tile << kTileLog;
+      if (!ABS)
+        for (int j = threadIdx.x; j < kTileCols; j += kSymThreads) xc[j] = k0 + j < nx ? (double)xP[k0 + j] : 0.0;
+      __syncthreads();
+      run(at + len * wave / kSymWaves, at + len * (wave + 1) / kSymWaves, true);
+      __syncthreads();
+      for (int j = threadIdx.x; j < kTileCols; j += kSymThreads) {
+        const unsigned long long a = yc[j];
+        if (a != 0ull) {
+          atomicAdd(&yT[k0 + j], a);
+          yc[j] = 0ull;
+        }
       }
-      if (tile != cur) {
-        if (cur != 0xffffffffu) flush(cur);
-        cur = tile;
-      }
-      if (valid) atomicAdd(&ya[wave][col], q);
+      at = to;
     }
   }
-  if (cur != 0xffffffffu) flush(cur);
   __syncthreads();
-  for (int t = threadIdx.x; t < kTileRows; t += kBlock)
-    if (m0 + t < n && yr[t] != 0ull) atomicAdd(&yT[m0 + t], yr[t]);
+  for (int j = threadIdx.x; j < kSymRows; j += kSymThreads)
+    if (yr[j] != 0ull) atomicAdd(&yT[m0 + j], yr[j]);
 }
 
 // y[I] = diag[I] x[I] + 2^e (yT[pos[I]] (+ yT[n + bPos[I]] with split
@@ -2334,11 +2502,13 @@ __global__ void kSymFinish(const double* __restrict__ diag, const double* __rest
                            const unsigned long long* __restrict__ yT, const unsigned long long* __restrict__ bound,
                            const uint32_t* __restrict__ pos, const uint32_t* __restrict__ bPos, int64_t n,
                            int64_t nx) {
-  const int e = symFixExp(yT, nx, bound);
+  const double range = symFixRange(yT, nx, bound);
+  const int e = symFixExp(range);
+  const bool none = isinf(range);  // no fixed point holds the sums
   for (int64_t I = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; I < n; I += (int64_t)gridDim.x * blockDim.x) {
     long long t = (long long)yT[pos[I]];
     if (bPos) t += (long long)yT[n + bPos[I]];
-    y[I] = fma(diag[I], x[I], ldexp((double)t, e));
+    y[I] = none ? (double)NAN : fma(diag[I], x[I], ldexp((double)t, e));
   }
 }
 
@@ -2358,7 +2528,7 @@ __global__ void kGatherPermMax(const double* __restrict__ x, const uint32_t* __r
   double m = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nx; i += (int64_t)gridDim.x * blockDim.x) {
     const double v = x[i < n ? perm[i] : bPerm[i - n]];
-    xP[i] = (XT)v;
+    xP[i] = fabs(v) <= DBL_MAX ? (XT)v : (XT)0;  // (with an infinite max|x| kSymFinish makes every sum NaN)
     m = fmax(m, fabs(v));
   }
 #pragma unroll
@@ -2374,32 +2544,15 @@ __global__ void kGatherPermMax(const double* __restrict__ x, const uint32_t* __r
   }
 }
 
-// off-diagonal row sums of |H| over a stored half grown by rows
-// [nOld, n): row I's stored entries add into acc[I] and each into its
-// column's acc[J]; every |v| is rounded up to a multiple of 2^-32 and
-// summed as an integer (exactly, so in any order).  One wave per row.
-template <typename VT>
-__global__ void kRowAbsSum(const int64_t* __restrict__ rowPtr, const int32_t* __restrict__ cols,
-                           const VT* __restrict__ vals, int64_t nOld, int64_t n, unsigned long long* acc) {
-  const int lane = __lane_id();
-  for (int64_t I = nOld + ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / 64; I < n;
-       I += ((int64_t)gridDim.x * blockDim.x) / 64) {
-    unsigned long long r = 0ull;
-    for (int64_t p = rowPtr[I] + lane; p < rowPtr[I + 1]; p += 64) {
-      const unsigned long long q = (unsigned long long)ceil(ldexp(fabs((double)vals[p]), 32));
-      atomicAdd(&acc[cols[p]], q);
-      r += q;
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) r += __shfl_xor(r, o, 64);
-    if (lane == 0 && r) atomicAdd(&acc[I], r);
-  }
-}
-
-__global__ void kMaxU64(const unsigned long long* __restrict__ a, int64_t n, unsigned long long* out) {
+// the largest sum of a row: a[pos[I]] (+ a[n + bPos[I]] with split columns)
+__global__ void kMaxU64(const unsigned long long* __restrict__ a, const uint32_t* __restrict__ pos,
+                        const uint32_t* __restrict__ bPos, int64_t n, unsigned long long* out) {
   unsigned long long m = 0ull;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    m = a[i] > m ? a[i] : m;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    unsigned long long t = a[pos[i]];
+    if (bPos) t += a[n + bPos[i]];
+    m = t > m ? t : m;
+  }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     const unsigned long long t = __shfl_xor(m, o, 64);
@@ -3272,12 +3425,22 @@ void launchTrevUnpack(const double* ci, int64_t n, int nroots, int64_t ld, const
   HIP_CHECK(hipGetLastError());
 }
 
-static int computeUnits();
 
 void launchIota(uint32_t* v, int64_t n, hipStream_t s) {
   if (n <= 0) return;
   kIota<<<gridFor(n, kBlock, 8192), kBlock, 0, s>>>(v, n);
   HIP_CHECK(hipGetLastError());
+}
+
+static int computeUnits() {
+  static int cus = 0;
+  if (cus == 0) {
+    int dev = 0;
+    HIP_CHECK(hipGetDevice(&dev));
+    HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    if (cus <= 0) cus = 256;
+  }
+  return cus;
 }
 
 void launchPtReduce(const DevSystem& S, const uint64_t* keys, const uint32_t* idx, const double* num, int64_t m,
@@ -3674,17 +3837,6 @@ void launchPermRowsF32(const int64_t* rowPtr, const int32_t* cols, const float* 
   HIP_CHECK(hipGetLastError());
 }
 
-static int computeUnits() {
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0;
-    HIP_CHECK(hipGetDevice(&dev));
-    HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    if (cus <= 0) cus = 256;
-  }
-  return cus;
-}
-
 void* XScratch::get(size_t bytes) const {
   if (mem) {
     mem->reserve(bytes);
@@ -3797,26 +3949,29 @@ void launchSigmaPermF32(const int64_t* rp, const int32_t* cols, const float* val
 
 void TiledHam::release() {
   for (DevMem* m : {&segBase, &segTile, &segCnt, &segStart, &segInst, &segTotal, &fill, &blockE, &blockI, &idx, &vals,
-                    &lo, &inst})
+                    &lo, &inst, &order, &blockOf, &bigI, &smallI, &lead, &groups, &symInst, &unitStart, &units})
     m->release();
   n = -1;
   hasLo = false;
 }
 
+// the half-storage sigma's order of a tiled copy and its work units
+static void buildSymOrder(TiledHam& T, int bigMin, Workspace& ws, hipStream_t s);
+
 size_t tiledHamBytes(int64_t n, int64_t nnz, bool f32) {
   const int64_t blocks = (n + kTileRows - 1) / kTileRows;
   // entries, one instruction per 32 entries at most on average plus one per
-  // segment, segment tables (48 bytes) with at most one segment per 64
-  // entries or per block
+  // segment (twice: the half-storage sigma's order), segment tables (88
+  // bytes) with at most one segment per 64 entries or per block
   const int64_t segs = nnz / 64 + blocks;
-  return (size_t)nnz * (4 + (f32 ? 4 : 8)) + (size_t)(nnz / 32 + segs) * 8 + (size_t)segs * 48 +
-         (size_t)(blocks + 1) * 24;
+  return (size_t)nnz * (4 + (f32 ? 4 : 8)) + (size_t)(nnz / 32 + segs) * 16 + (size_t)segs * 88 +
+         (size_t)(blocks + 1) * 40;
 }
 
 bool buildTiledHam(TiledHam& T, const int64_t* rowPtr, const int32_t* cols, const double* vals64,
                    const float* vals32, const uint32_t* perm, const uint32_t* pos, const uint32_t* bIdx,
                    const uint32_t* bPos, int64_t n, int64_t nnz, Workspace& ws, hipStream_t s, bool splitCols,
-                   int stageMin, const float* valsLo) {
+                   int stageMin, const float* valsLo, bool sym) {
   T.n = -1;
   T.hasLo = false;
   if (n <= 0) return false;
@@ -3898,6 +4053,7 @@ bool buildTiledHam(TiledHam& T, const int64_t* rowPtr, const int32_t* cols, cons
   T.f32 = f32;
   T.split = split;
   T.hasLo = withLo;
+  if (sym) buildSymOrder(T, stageMin, ws, s);
   return true;
 }
 
@@ -3953,6 +4109,56 @@ void launchSigmaTiled(const TiledHam& T, const double* diag, const uint32_t* per
   HIP_CHECK(hipGetLastError());
 }
 
+// the half-storage sigma's order of a tiled copy and its work units
+static void buildSymOrder(TiledHam& T, int bigMin, Workspace& ws, hipStream_t s) {
+  const int64_t S = T.segments, supers = (T.blocks + kSymBlocks - 1) / kSymBlocks;
+  if (T.instructions >= 0xffffffffLL) throw HipError("tiled Hamiltonian: too many instructions");
+  T.order.reserve((size_t)std::max<int64_t>(S, 1) * 4);
+  T.blockOf.reserve((size_t)std::max<int64_t>(S, 1) * 4);
+  for (DevMem* m : {&T.bigI, &T.smallI, &T.lead}) {
+    m->reserve((size_t)(S + 1) * 8);
+    HIP_CHECK(hipMemsetAsync(m->as<int64_t>() + S, 0, 8, s));
+  }
+  T.groups.reserve((size_t)(S + 1) * 8);
+  T.symInst.reserve((size_t)std::max<int64_t>(T.instructions, 1) * 8);
+  T.unitStart.reserve((size_t)(supers + 1) * 8);
+  const int64_t* segBase = T.segBase.as<int64_t>();
+  kSymRank<<<gridFor(S), kBlock, 0, s>>>(segBase, T.blocks, S, T.segTile.as<uint32_t>(), T.segTotal.as<uint32_t>(),
+                                         (uint32_t)bigMin, T.order.as<uint32_t>(), T.blockOf.as<uint32_t>(),
+                                         T.bigI.as<int64_t>(), T.smallI.as<int64_t>(), T.lead.as<int64_t>());
+  HIP_CHECK(hipGetLastError());
+  for (DevMem* m : {&T.bigI, &T.smallI, &T.lead}) exclusiveScanI64(m->as<int64_t>(), S + 1, ws, s);
+  kSymEmit<<<gridFor(S), kBlock, 0, s>>>(S, T.order.as<uint32_t>(), T.blockOf.as<uint32_t>(), T.blockE.as<int64_t>(),
+                                         T.segTile.as<uint32_t>(), T.segTotal.as<uint32_t>(),
+                                         T.segStart.as<uint32_t>(), T.bigI.as<int64_t>(), T.smallI.as<int64_t>(),
+                                         T.lead.as<int64_t>(), T.symInst.as<uint2>(), T.groups.as<uint2>());
+  HIP_CHECK(hipGetLastError());
+  // Units of I / (8 CUs) instructions: two workgroups for each of the four
+  // that a CU holds, between 64 (two steps for each wave) and 1,024; 57,963
+  // determinants of 40 orbitals: 89 us in the 190 this gives, 95 in units of
+  // 512, 128 of 1,024; 1,000,003 of 24 orbitals: 1,790 us in units of 256,
+  // 1,711 of 512, 1,713 of 1,024, 1,701 of 2,048.
+  const int64_t per = std::min<int64_t>(1024, std::max<int64_t>(64, T.instructions / ((int64_t)computeUnits() * 8)));
+  T.unitCap = 2 * supers + T.instructions / per;
+  T.units.reserve((size_t)T.unitCap * sizeof(SymUnit));
+  kSymUnits<<<gridFor(supers), kBlock, 0, s>>>(segBase, T.blocks, supers, S, T.bigI.as<int64_t>(),
+                                               T.smallI.as<int64_t>(), T.lead.as<int64_t>(), T.groups.as<uint2>(),
+                                               per, T.unitStart.as<int64_t>(), nullptr, 0);
+  exclusiveScanI64(T.unitStart.as<int64_t>(), supers + 1, ws, s);
+  kSymUnits<<<gridFor(supers), kBlock, 0, s>>>(segBase, T.blocks, supers, S, T.bigI.as<int64_t>(),
+                                               T.smallI.as<int64_t>(), T.lead.as<int64_t>(), T.groups.as<uint2>(),
+                                               per, T.unitStart.as<int64_t>(), T.units.as<SymUnit>(), T.unitCap);
+  HIP_CHECK(hipGetLastError());
+}
+
+template <typename VT, typename XT, bool LO, bool ABS>
+static void runSymTiles(const TiledHam& T, int64_t nx, const XT* xs, unsigned long long* yT,
+                        const unsigned long long* bound, hipStream_t s) {
+  kSigmaTiledSym<VT, XT, LO, ABS><<<(unsigned)T.unitCap, kSymThreads, 0, s>>>(
+      T.units.as<SymUnit>(), T.symInst.as<uint2>(), T.groups.as<uint2>(), T.blockE.as<int64_t>(),
+      T.idx.as<uint32_t>(), T.vals.as<VT>(), LO ? T.lo.as<float>() : nullptr, T.n, nx, xs, yT, bound);
+}
+
 void launchSigmaTiledSym(const TiledHam& T, const double* diag, const uint32_t* perm, const uint32_t* bPerm,
                          const uint32_t* pos, const uint32_t* bPos, const double* x, double* y, const XScratch& xP,
                          unsigned long long* yT, const unsigned long long* bound, hipStream_t s, bool exact) {
@@ -3962,41 +4168,34 @@ void launchSigmaTiledSym(const TiledHam& T, const double* diag, const uint32_t* 
     throw HipError("tiled sigma: split columns need the beta-major order");
   if (exact && T.f32 && !T.hasLo) throw HipError("tiled sigma: the exact FP32 form needs the lo values");
   const int64_t nx = bPerm ? 2 * n : n;
-  const unsigned grid = (unsigned)T.blocks;
   kFillZeroU64<<<gridFor(nx + 1), kBlock, 0, s>>>(yT, nx + 1);
   if (T.f32 && !exact) {
     float* xs = (float*)xP.get((size_t)nx * 4);
     kGatherPermMax<float><<<gridFor(nx, kBlock, 1024), kBlock, 0, s>>>(x, perm, bPerm, n, xs, yT + nx);
-    kSigmaTiledSym<float, float, 8, false><<<grid, kBlock, 0, s>>>(
-        T.inst.as<uint2>(), T.blockI.as<int64_t>(), T.blockE.as<int64_t>(), T.idx.as<uint32_t>(), T.vals.as<float>(),
-        nullptr, n, nx, xs, yT, bound);
+    runSymTiles<float, float, false, false>(T, nx, xs, yT, bound, s);
   } else {
     double* xs = (double*)xP.get((size_t)nx * 8);
     kGatherPermMax<double><<<gridFor(nx, kBlock, 1024), kBlock, 0, s>>>(x, perm, bPerm, n, xs, yT + nx);
     if (T.f32)  // the exact FP32 form: hi + lo values, x in FP64
-      kSigmaTiledSym<float, double, 8, true><<<grid, kBlock, 0, s>>>(
-          T.inst.as<uint2>(), T.blockI.as<int64_t>(), T.blockE.as<int64_t>(), T.idx.as<uint32_t>(),
-          T.vals.as<float>(), T.lo.as<float>(), n, nx, xs, yT, bound);
+      runSymTiles<float, double, true, false>(T, nx, xs, yT, bound, s);
     else
-      kSigmaTiledSym<double, double, 8, false><<<grid, kBlock, 0, s>>>(
-          T.inst.as<uint2>(), T.blockI.as<int64_t>(), T.blockE.as<int64_t>(), T.idx.as<uint32_t>(),
-          T.vals.as<double>(), nullptr, n, nx, xs, yT, bound);
+      runSymTiles<double, double, false, false>(T, nx, xs, yT, bound, s);
   }
   kSymFinish<<<gridFor(n), kBlock, 0, s>>>(diag, x, y, yT, bound, pos, bPos, n, nx);
   HIP_CHECK(hipGetLastError());
 }
 
-void launchSymRowBound(const int64_t* rowPtr, const int32_t* cols, const double* vals64, const float* vals32,
-                       int64_t nOld, int64_t n, unsigned long long* acc, unsigned long long* bound, hipStream_t s) {
-  if (n > nOld) kFillZeroU64<<<gridFor(n - nOld), kBlock, 0, s>>>(acc + nOld, n - nOld);
+void launchSymRowBound(const TiledHam& T, const uint32_t* pos, const uint32_t* bPos, unsigned long long* yT,
+                       unsigned long long* bound, hipStream_t s) {
+  const int64_t n = T.n, nx = bPos ? 2 * n : n;
+  if (n <= 0) return;
+  kFillZeroU64<<<gridFor(nx), kBlock, 0, s>>>(yT, nx);
   kFillZeroU64<<<1, 64, 0, s>>>(bound, 1);
-  if (n > nOld) {
-    if (vals32)
-      kRowAbsSum<float><<<gridFor(n - nOld, kWaves), kBlock, 0, s>>>(rowPtr, cols, vals32, nOld, n, acc);
-    else
-      kRowAbsSum<double><<<gridFor(n - nOld, kWaves), kBlock, 0, s>>>(rowPtr, cols, vals64, nOld, n, acc);
-  }
-  if (n > 0) kMaxU64<<<gridFor(n, kBlock, 1024), kBlock, 0, s>>>(acc, n, bound);
+  if (T.f32)
+    runSymTiles<float, float, false, true>(T, nx, nullptr, yT, nullptr, s);
+  else
+    runSymTiles<double, double, false, true>(T, nx, nullptr, yT, nullptr, s);
+  kMaxU64<<<gridFor(n, kBlock, 1024), kBlock, 0, s>>>(yT, pos, bPos, n, bound);
   kU64ScaledToDouble<<<1, 64, 0, s>>>(bound);
   HIP_CHECK(hipGetLastError());
 }

@@ -1,0 +1,51 @@
+"""Kernels at the sizes where their work split changes (partial tiles, few or
+many work units, remainders), against the oracle."""
+import numpy as np
+import pytest
+
+import helpers
+from oracle_bind import OracleSystem
+
+pytestmark = pytest.mark.gpu
+
+
+def _space(path, occ, n, W):
+    o = OracleSystem(path)
+    dets = helpers.occ_to_det(occ, W)[None, :]
+    eps = 1e-2
+    while len(dets) < n:
+        new = o.screen(dets, np.ones(len(dets)), eps)
+        if len(new):
+            dets = np.concatenate([dets, new])
+        eps *= 0.5
+    return dets[:n]
+
+
+def _system(case, tmp_path):
+    from dice_amd import synth
+    path = str(tmp_path / "FCIDUMP")
+    if case == "w1":
+        synth.write_molecular_fcidump(path, 0, 16, 8, 8, 64)
+        return path, synth.hf_occupation(8, 8), 1
+    synth.write_molecular_fcidump(path, 5, 34, 6, 6, 12)
+    return path, synth.hf_occupation(6, 6), 2
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("case,n", [("w1", 1), ("w1", 2), ("w1", 255), ("w1", 257), ("w1", 6001), ("w2", 1025)])
+def test_sigma_work_units(case, n, prec, tmp_path):
+    """Blocks without entries, of less than one unit and of many units.  Bar:
+    1e-12 of the largest element in FP64 (sums of about a thousand terms), 3e-6
+    with FP32 values and vectors (two roundings of 2^-24 a term)."""
+    from dice_amd import shci
+    path, occ, W = _system(case, tmp_path)
+    dets = _space(path, occ, n, W)
+    s = shci.System.from_fcidump(path)
+    s.set_options(precision=prec)
+    s.set_dets(dets)
+    s.make_hamiltonian()
+    o = OracleSystem(path)
+    o.csr_append(dets)
+    x = np.random.default_rng(n).normal(size=n)
+    yo = o.sigma(x)
+    assert np.max(np.abs(s.hmult(x) - yo)) <= (3e-6 if prec else 1e-12) * np.max(np.abs(yo))
