@@ -267,6 +267,10 @@ DevSystem Engine::ptSystem() const {
   return P;
 }
 
+void Engine::ptTables() {
+  if (!ptDense[0].p) buildDenseHeatBath(S, ptDense, stream);
+}
+
 double Engine::ptDeterministic(const double* dCi, double e0, double eps2, double* psi1Norm, int64_t* nExternal,
                                int* nPartitions) {
   const int W = hs.W;
@@ -275,17 +279,20 @@ double Engine::ptDeterministic(const double* dCi, double e0, double eps2, double
   uint32_t nparts = 1;
   if (n > 0) {
     ensureTable(n);
+    ptTables();
     const DevSystem P = ptSystem();
-    ptCounts.reserve((size_t)(n + 1) * 8);
+    const int slices = ptSlices(n, hs.nelec);
+    const int64_t nc = n * slices;
+    ptCounts.reserve((size_t)(nc + 1) * 8);
     int64_t* cnt = ptCounts.as<int64_t>();
-    // per-source candidate counts of one partition, scanned into offsets
+    // candidate counts of one partition, scanned into offsets
     auto countPass = [&](uint32_t parts, uint32_t part) {
-      HIP_CHECK(hipMemsetAsync(cnt + n, 0, 8, stream));
-      launchPtGen(P, dets.as<uint64_t>(), n, dCi, eps2, table.as<int32_t>(), slots, parts, part, cnt, nullptr,
-                  nullptr, nullptr, stream);
-      exclusiveScanI64(cnt, n + 1, ws, stream);
+      HIP_CHECK(hipMemsetAsync(cnt + nc, 0, 8, stream));
+      launchPtGen(P, dets.as<uint64_t>(), n, dCi, eps2, table.as<int32_t>(), slots, parts, part, slices, ptDense, cnt,
+                  nullptr, nullptr, nullptr, stream);
+      exclusiveScanI64(cnt, nc + 1, ws, stream);
       int64_t total = 0;
-      HIP_CHECK(hipMemcpyAsync(&total, cnt + n, 8, hipMemcpyDeviceToHost, stream));
+      HIP_CHECK(hipMemcpyAsync(&total, cnt + nc, 8, hipMemcpyDeviceToHost, stream));
       HIP_CHECK(hipStreamSynchronize(stream));
       return total;
     };
@@ -306,8 +313,8 @@ double Engine::ptDeterministic(const double* dCi, double e0, double eps2, double
       ptKeys.reserve((size_t)m * W * 8);
       ptNum.reserve((size_t)m * 8);
       ptIdx.reserve((size_t)m * 4);
-      launchPtGen(P, dets.as<uint64_t>(), n, dCi, eps2, table.as<int32_t>(), slots, nparts, part, nullptr, cnt,
-                  ptKeys.as<uint64_t>(), ptNum.as<double>(), stream);
+      launchPtGen(P, dets.as<uint64_t>(), n, dCi, eps2, table.as<int32_t>(), slots, nparts, part, slices, ptDense,
+                  nullptr, cnt, ptKeys.as<uint64_t>(), ptNum.as<double>(), stream);
       launchIota(ptIdx.as<uint32_t>(), m, stream);
       radixSortKeys(ptKeys.as<uint64_t>(), ptIdx.as<uint32_t>(), m, W, hs.nso, true, ws, stream);
       launchPtReduce(P, ptKeys.as<uint64_t>(), ptIdx.as<uint32_t>(), ptNum.as<double>(), m, e0, ptPartial, ptStartCnt,
@@ -375,8 +382,10 @@ double Engine::ptSemistochastic(const double* dCi, double e0, double eps2, doubl
   std::vector<double> wts(Nmc, 0.0);
   std::vector<uint32_t> src32;
   ensureTable(n);
+  ptTables();
   const DevSystem P = ptSystem();
-  ptCounts.reserve((size_t)(Nmc + 1) * 8);
+  const int slices = ptSlices(Nmc, hs.nelec);
+  ptCounts.reserve(((size_t)Nmc * slices + 1) * 8);
   ptOut.reserve(64);
   int64_t* cnt = ptCounts.as<int64_t>();
   if (log) fprintf(log, "%6s  %18s  %5s %18s %10s  %10s\n", "Iter", "EPTcurrent", "State", "EPTavg", "Error", "Time(s)");
@@ -408,13 +417,14 @@ double Engine::ptSemistochastic(const double* dCi, double e0, double eps2, doubl
     ptW.reserve((size_t)std::max(distinct, 1) * 8);
     HIP_CHECK(hipMemcpyAsync(ptSrc.p, src32.data(), (size_t)distinct * 4, hipMemcpyHostToDevice, stream));
     HIP_CHECK(hipMemcpyAsync(ptW.p, wts.data(), (size_t)distinct * 8, hipMemcpyHostToDevice, stream));
-    HIP_CHECK(hipMemsetAsync(cnt + distinct, 0, 8, stream));
+    const int64_t nc = (int64_t)distinct * slices;
+    HIP_CHECK(hipMemsetAsync(cnt + nc, 0, 8, stream));
     launchPtGenStoch(P, dets.as<uint64_t>(), ptSrc.as<uint32_t>(), ptW.as<double>(), distinct, dCi, eps2, eps2Large,
-                     (double)Nmc, table.as<int32_t>(), slots, cnt, nullptr, nullptr, nullptr, nullptr, nullptr,
-                     stream);
-    exclusiveScanI64(cnt, distinct + 1, ws, stream);
+                     (double)Nmc, table.as<int32_t>(), slots, slices, ptDense, cnt, nullptr, nullptr, nullptr, nullptr,
+                     nullptr, stream);
+    exclusiveScanI64(cnt, nc + 1, ws, stream);
     int64_t m = 0;
-    HIP_CHECK(hipMemcpyAsync(&m, cnt + distinct, 8, hipMemcpyDeviceToHost, stream));
+    HIP_CHECK(hipMemcpyAsync(&m, cnt + nc, 8, hipMemcpyDeviceToHost, stream));
     HIP_CHECK(hipStreamSynchronize(stream));
     if (m > INT32_MAX) throw std::invalid_argument("semistochastic PT: more than 2^31 candidates in one iteration");
     double host[2] = {0.0, 0.0};
@@ -425,12 +435,13 @@ double Engine::ptSemistochastic(const double* dCi, double e0, double eps2, doubl
       ptP.reserve((size_t)m);
       ptIdx.reserve((size_t)m * 4);
       launchPtGenStoch(P, dets.as<uint64_t>(), ptSrc.as<uint32_t>(), ptW.as<double>(), distinct, dCi, eps2,
-                       eps2Large, (double)Nmc, table.as<int32_t>(), slots, nullptr, cnt, ptKeys.as<uint64_t>(),
-                       ptNum.as<double>(), ptN2.as<double>(), ptP.as<uint8_t>(), stream);
+                       eps2Large, (double)Nmc, table.as<int32_t>(), slots, slices, ptDense, nullptr, cnt,
+                       ptKeys.as<uint64_t>(), ptNum.as<double>(), ptN2.as<double>(), ptP.as<uint8_t>(), stream);
       launchIota(ptIdx.as<uint32_t>(), m, stream);
       radixSortKeys(ptKeys.as<uint64_t>(), ptIdx.as<uint32_t>(), m, W, hs.nso, true, ws, stream);
       launchPtStochReduce(P, ptKeys.as<uint64_t>(), ptIdx.as<uint32_t>(), ptNum.as<double>(), ptN2.as<double>(),
-                          ptP.as<uint8_t>(), m, e0, (double)Nmc, ptPartial, ptOut.as<double>(), stream);
+                          ptP.as<uint8_t>(), m, e0, (double)Nmc, ptPartial, ptStartCnt, ptStarts, ws,
+                          ptOut.as<double>(), stream);
       HIP_CHECK(hipMemcpyAsync(host, ptOut.p, 16, hipMemcpyDeviceToHost, stream));
       HIP_CHECK(hipStreamSynchronize(stream));
     }

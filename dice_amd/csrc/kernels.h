@@ -28,27 +28,30 @@ void launchCmax(const double* ci, int nroots, int64_t ld, int64_t n, double* cma
 // Screens the source determinants [begin, end) of `dets` (the whole
 // variational space is probed for membership).
 // Deterministic EN-PT2 candidates of sources [0, n) (SHCI/SHCIgetdeterminants.cpp:40-171):
-// with fillStart == nullptr the count pass writes counts[src]; otherwise the
-// fill pass writes each source's candidates (determinants outD, numerators
-// H_ai c_i outN) from fillStart[src] in the reference's generation order.
+// each cut into `slices` parts (ptSlices): with fillStart == nullptr the count
+// pass writes counts[src * slices + part]; otherwise the fill pass writes each
+// part's candidates (determinants outD, numerators H_ai c_i outN) from
+// fillStart on, a source's by electron pairs as the reference generates them.
 // Only candidates outside the membership table and in partition `part` of
-// `nparts` are kept.
+// `nparts` are kept.  dense: buildDenseHeatBath's two tables.
+int ptSlices(int64_t nsrc, int nelec);
+void buildDenseHeatBath(const DevSystem& S, DevMem* dense, hipStream_t s);
 void launchPtGen(const DevSystem& S, const uint64_t* dets, int64_t n, const double* ci, double eps2,
-                 const int32_t* table, uint64_t slots, uint32_t nparts, uint32_t part, int64_t* counts,
-                 const int64_t* fillStart, uint64_t* outD, double* outN, hipStream_t s);
+                 const int32_t* table, uint64_t slots, uint32_t nparts, uint32_t part, int slices, const DevMem* dense,
+                 int64_t* counts, const int64_t* fillStart, uint64_t* outD, double* outN, hipStream_t s);
 // Semistochastic PT candidates of the sampled sources src[0..nsrc) with
 // weights w (count pass when fillStart == nullptr): numerators H_ai w, second
 // moments H_ai^2 w (w nmc/(nmc-1) - c) and the epsilon2Large flag
 // (SHCI/SHCIgetdeterminants.cpp:889-1046), in generation order
 void launchPtGenStoch(const DevSystem& S, const uint64_t* dets, const uint32_t* src, const double* w, int64_t nsrc,
                       const double* ci, double eps2, double eps2Large, double nmc, const int32_t* table, uint64_t slots,
-                      int64_t* counts, const int64_t* fillStart, uint64_t* outD, double* outN, double* outN2,
-                      uint8_t* outP, hipStream_t s);
+                      int slices, const DevMem* dense, int64_t* counts, const int64_t* fillStart, uint64_t* outD,
+                      double* outN, double* outN2, uint8_t* outP, hipStream_t s);
 // out[0..1] (device) = the two energy sums of one semistochastic iteration
 // over m candidates sorted by determinant (payload idx)
 void launchPtStochReduce(const DevSystem& S, const uint64_t* keys, const uint32_t* idx, const double* num,
                          const double* num2, const uint8_t* pres, int64_t m, double e0, double nmc, DevMem& partial,
-                         double* out, hipStream_t s);
+                         DevMem& counts, DevMem& starts, Workspace& ws, double* out, hipStream_t s);
 // time reversal: flags + scan of the open-shell determinants among
 // dets[i0, i1); with block, the block of the plain basis E for them (the
 // i1 - i0 determinants, then the flipped copies of the open-shell ones) to

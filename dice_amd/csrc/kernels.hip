@@ -388,24 +388,53 @@ struct PtStoch {
   uint8_t* outP;
 };
 
+// a dense copy of one spin case's heat-bath lists (cleared to NaN first)
+__global__ void kFillNan(float* v, int64_t m) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x)
+    v[i] = NAN;
+}
+__global__ void kDenseHeatBath(const float* val, const uint32_t* pair, const int64_t* start, int64_t npair, int norb,
+                               float* dense) {
+  for (int64_t p = blockIdx.x; p < npair; p += gridDim.x)
+    for (int64_t k = start[p] + threadIdx.x; k < start[p + 1]; k += blockDim.x)
+      dense[p * norb * norb + (int64_t)(pair[k] & 0xFFFF) * norb + (pair[k] >> 16)] = val[k];
+}
+
 // Candidates D_a of sources [0, ndets) with numerator H_ai c_i: singles with
 // |Hij_1Excite| > eps, doubles while the float heat-bath value passes eps
 // (numerator = value x parity of the excitation x c_i), eps = |eps2 / c_i|,
 // no active-space limits, the PT restrictions in S; kept when D_a is not a
 // variational determinant and falls in partition `part`.
+//
+// Work: a source's pairs of electrons are cut into `slices` parts (with more
+// than one, part 0 is the singles), a wave each, so that a few sources fill
+// the chip too.  A pair's doubles are found in one of two ways, whichever
+// looks at fewer places: the prefix of the pair's |v|-sorted list that passes
+// eps, most of whose entries excite into occupied orbitals, or every pair of
+// open orbitals, whose values a dense copy of the lists gives (dense[same
+// spin][pair][a n + b], NaN where the list has no entry).
+// Measured: 200 sampled sources of 57,963 determinants of 40 orbitals (eps2
+// 3e-4), count and fill 33 + 41 -> 0.71 + 0.89 ms with the parts; 27,685
+// sources of 24 orbitals (eps2 3e-4, 33 million determinants found), one part
+// each, 12.6 + 14.8 -> 7.5 + 8.8 ms with the open pairs: there the membership
+// probes bound it.
 template <int W, bool FILL, bool STOCH>
 __global__ void __launch_bounds__(kBlock) kPtGen(DevSystem S, const uint64_t* dets, int64_t ndets, const double* ci,
                                                  double eps2, const int32_t* table, uint64_t mask, uint32_t nparts,
                                                  uint32_t part, int64_t* counts, const int64_t* fillStart,
-                                                 uint64_t* outD, double* outN, PtStoch st) {
+                                                 uint64_t* outD, double* outN, PtStoch st, int slices,
+                                                 const float* __restrict__ dense0, const float* __restrict__ dense1) {
   __shared__ uint8_t sClosed[kWaves][128];
   __shared__ uint8_t sOpen[kWaves][128];
+  __shared__ uint8_t sSpin[kWaves][2][64];  // open spatial orbitals of each spin
   __shared__ int sExcl[kWaves][65];
   __shared__ int64_t sStart[kWaves][64];
   __shared__ int sPair[kWaves][64];
   const int wave = threadIdx.x >> 6, lane = __lane_id();
-  const int nso = S.nso;
-  for (int64_t di = (int64_t)blockIdx.x * kWaves + wave; di < ndets; di += (int64_t)gridDim.x * kWaves) {
+  const int nso = S.nso, norb = S.norb;
+  for (int64_t wi = (int64_t)blockIdx.x * kWaves + wave; wi < ndets * slices; wi += (int64_t)gridDim.x * kWaves) {
+    const int64_t di = wi / slices;
+    const int slice = (int)(wi - di * slices);
     const int64_t src = STOCH ? (int64_t)st.src[di] : di;
     uint64_t d[W];
 #pragma unroll
@@ -416,7 +445,7 @@ __global__ void __launch_bounds__(kBlock) kPtGen(DevSystem S, const uint64_t* de
     const double epsL = STOCH ? __ddiv_rn(st.eps2Large, fabs(c)) : 0.0;
     const double wfac = STOCH ? __dsub_rn(__ddiv_rn(__dmul_rn(wt, st.nmc), st.nmc - 1.0), c) : 0.0;
     PtSink<W, FILL> sink;
-    sink.pos = FILL ? fillStart[di] : 0;
+    sink.pos = FILL ? fillStart[wi] : 0;
     sink.cnt = 0;
     sink.outD = outD;
     sink.outN = outN;
@@ -433,6 +462,14 @@ __global__ void __launch_bounds__(kBlock) kPtGen(DevSystem S, const uint64_t* de
       nclosed += __popcll(mc);
       nopen += __popcll(mo);
     }
+    int nSpin[2];
+#pragma unroll
+    for (int sp = 0; sp < 2; sp++) {  // (at most 63 spatial orbitals)
+      const bool o = lane < norb && !occ<W>(d, 2 * lane + sp);
+      const uint64_t mo = __ballot(o);
+      if (o) sSpin[wave][sp][__popcll(mo & lanemaskLt())] = (uint8_t)lane;
+      nSpin[sp] = __popcll(mo);
+    }
     __syncwarp();
     int cur[SHCI_MAX_RESTRICT];
     for (int r = 0; r < S.nrestrict; r++) {
@@ -441,7 +478,7 @@ __global__ void __launch_bounds__(kBlock) kPtGen(DevSystem S, const uint64_t* de
       cur[r] = cc;
     }
     // ---- single excitations
-    const int nsingle = nclosed * nopen;
+    const int nsingle = slice == 0 ? nclosed * nopen : 0;
     for (int t0 = 0; t0 < nsingle; t0 += 64) {
       int t = t0 + lane;
       bool keep = false, pres = false;
@@ -475,11 +512,14 @@ __global__ void __launch_bounds__(kBlock) kPtGen(DevSystem S, const uint64_t* de
     // ---- double excitations
     if (!(S.maxEntryAbs < eps)) {
       const int npairs = nclosed * (nclosed - 1) / 2;
-      for (int p0 = 0; p0 < npairs; p0 += 64) {
+      const int perSlice = slices > 1 ? (npairs + slices - 2) / (slices - 1) : npairs;
+      const int pBegin = slices > 1 ? (slice == 0 ? npairs : (slice - 1) * perSlice) : 0;
+      const int pEnd = pBegin + perSlice < npairs ? pBegin + perSlice : npairs;
+      for (int p0 = pBegin; p0 < pEnd; p0 += 64) {
         int p = p0 + lane;
         int len = 0;
         int64_t st = 0;
-        if (p < npairs) {
+        if (p < pEnd) {
           int i = (int)((1.0 + sqrt(1.0 + 8.0 * (double)p)) * 0.5);
           while (i * (i - 1) / 2 > p) i--;
           while ((i + 1) * i / 2 <= p) i++;
@@ -501,7 +541,13 @@ __global__ void __launch_bounds__(kBlock) kPtGen(DevSystem S, const uint64_t* de
           }
           len = (int)(lo - s0);
           st = s0;
-          sPair[wave][lane] = i | (j << 8) | (sameSpin << 16);
+          const int na = nSpin[cI & 1], all = sameSpin ? na * (na - 1) / 2 : na * nSpin[cJ & 1];
+          const bool direct = all < len;
+          if (direct) {
+            len = all;
+            st = (int64_t)pairIndex * norb * norb;
+          }
+          sPair[wave][lane] = i | (j << 8) | (sameSpin << 16) | (direct ? 1 << 17 : 0);
         }
         int inc = len;
 #pragma unroll
@@ -533,16 +579,41 @@ __global__ void __launch_bounds__(kBlock) kPtGen(DevSystem S, const uint64_t* de
             int pk = sPair[wave][q];
             int i = pk & 0xFF, j = (pk >> 8) & 0xFF, same = (pk >> 16) & 1;
             int cI = sClosed[wave][i], cJ = sClosed[wave][j];
-            int64_t idx = sStart[wave][q] + (k - sExcl[wave][q]);
-            uint32_t ab = S.hbPair[same][idx];
-            int a = 2 * (int)(ab & 0xFFFF) + (cI & 1), b = 2 * (int)(ab >> 16) + (cJ & 1);
+            const int kk = k - sExcl[wave][q];
+            int a, b;
+            float hv;
             bool ok = true;
+            if ((pk >> 17) & 1) {
+              int x, y;  // places in the lists of open orbitals: x > y for one spin
+              if (same) {
+                x = (int)((1.0f + sqrtf(1.0f + 8.0f * (float)kk)) * 0.5f);
+                while (x * (x - 1) / 2 > kk) x--;
+                while ((x + 1) * x / 2 <= kk) x++;
+                y = kk - x * (x - 1) / 2;
+              } else {
+                const int nb = nSpin[cJ & 1];
+                x = kk / nb;
+                y = kk - x * nb;
+              }
+              const int A = sSpin[wave][cI & 1][x], B = sSpin[wave][cJ & 1][y];
+              hv = (same ? dense1 : dense0)[sStart[wave][q] + A * norb + B];
+              ok = (double)fabsf(hv) >= eps;
+              a = 2 * A + (cI & 1);
+              b = 2 * B + (cJ & 1);
+            } else {
+              const int64_t idx = sStart[wave][q] + kk;
+              const uint32_t ab = S.hbPair[same][idx];
+              a = 2 * (int)(ab & 0xFFFF) + (cI & 1);
+              b = 2 * (int)(ab >> 16) + (cJ & 1);
+              ok = !(occ<W>(d, a) || occ<W>(d, b));
+              hv = ok ? S.hbVal[same][idx] : 0.0f;
+            }
             for (int r = 0; r < S.nrestrict && ok; r++) {
               const int8_t* m = S.rmult + r * nso;
               int e = cur[r] - m[cI] - m[cJ] + m[a] + m[b];
               if (e < S.rmin[r] || e > S.rmax[r]) ok = false;
             }
-            if (ok && !(occ<W>(d, a) || occ<W>(d, b))) {
+            if (ok) {
               cand[a >> 6] |= (1ull << (a & 63));
               cand[b >> 6] |= (1ull << (b & 63));
               cand[cI >> 6] &= ~(1ull << (cI & 63));
@@ -557,7 +628,6 @@ __global__ void __launch_bounds__(kBlock) kPtGen(DevSystem S, const uint64_t* de
               mid2[cI >> 6] |= (1ull << (cI & 63));
               nb += countBetween<W>(mid2, b < cJ ? b : cJ, b < cJ ? cJ : b);
               const double sgn = (nb & 1) ? -1.0 : 1.0;
-              const float hv = S.hbVal[same][idx];
               num = __dmul_rn(__dmul_rn((double)hv, sgn), wt);
               if (STOCH) {
                 num2 = __dmul_rn(__dmul_rn((double)__fmul_rn(hv, hv), wt), wfac);
@@ -575,7 +645,7 @@ __global__ void __launch_bounds__(kBlock) kPtGen(DevSystem S, const uint64_t* de
       int cc = sink.cnt;
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) cc += __shfl_xor(cc, o, 64);
-      if (lane == 0) counts[di] = cc;
+      if (lane == 0) counts[wi] = cc;
     }
   }
 }
@@ -2870,40 +2940,6 @@ __device__ __forceinline__ double* ptStageTables(const DevSystem& S) {
   return tab;
 }
 
-template <int W, bool LDS_TAB>
-__global__ void __launch_bounds__(kBlock) kPtStochReduce(DevSystem S, const uint64_t* keys, const uint32_t* idx,
-                                                         const double* num, const double* num2, const uint8_t* pres,
-                                                         int64_t m, double e0, double nmc, double* partial) {
-  const double* tab = ptStageTables<LDS_TAB>(S);
-  double sA = 0.0, sB = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x) {
-    if (i > 0 && detEqual<W>(keys + i * W, keys + (i - 1) * W)) continue;
-    double a1 = 0.0, a2 = 0.0, b1 = 0.0, b2 = 0.0;
-    for (int64_t j = i; j < m && detEqual<W>(keys + j * W, keys + i * W); j++) {
-      const uint32_t q = idx[j];
-      a1 = __dadd_rn(a1, num[q]);
-      a2 = __dadd_rn(a2, num2[q]);
-      if (pres[q]) {
-        b1 = __dadd_rn(b1, num[q]);
-        b2 = __dadd_rn(b2, num2[q]);
-      }
-    }
-    uint64_t d[W];
-#pragma unroll
-    for (int w = 0; w < W; w++) d[w] = keys[i * W + w];
-    const double den = __dsub_rn(ptEnergy<W, LDS_TAB>(S, tab, d), e0);
-    sA = __dadd_rn(sA, __ddiv_rn(__dsub_rn(__ddiv_rn(__dmul_rn(__dmul_rn(fabs(a1), fabs(a1)), nmc), nmc - 1.0), a2),
-                                 den));
-    sB = __dadd_rn(sB, __ddiv_rn(__dsub_rn(__ddiv_rn(__dmul_rn(__dmul_rn(fabs(b1), fabs(b1)), nmc), nmc - 1.0), b2),
-                                 den));
-  }
-  const double t0 = blockSum(sA), t1 = blockSum(sB);
-  if (threadIdx.x == 0) {
-    partial[2 * blockIdx.x] = t0;
-    partial[2 * blockIdx.x + 1] = t1;
-  }
-}
-
 __global__ void kIota(uint32_t* v, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     v[i] = (uint32_t)i;
@@ -2985,6 +3021,42 @@ __global__ void __launch_bounds__(kBlock) kPtReduceStarts(DevSystem S, const uin
   }
 }
 
+
+template <int W, bool LDS_TAB>
+__global__ void __launch_bounds__(kBlock) kPtStochReduce(DevSystem S, const uint64_t* keys, const uint32_t* idx,
+                                                         const double* num, const double* num2, const uint8_t* pres,
+                                                         const uint32_t* starts, const int64_t* nStarts, int64_t m,
+                                                         double e0, double nmc, double* partial) {
+  const double* tab = ptStageTables<LDS_TAB>(S);
+  double sA = 0.0, sB = 0.0;
+  const int64_t nu = *nStarts;
+  for (int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; u < nu; u += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t i = starts[u];
+    double a1 = 0.0, a2 = 0.0, b1 = 0.0, b2 = 0.0;
+    for (int64_t j = i; j < m && detEqual<W>(keys + j * W, keys + i * W); j++) {
+      const uint32_t q = idx[j];
+      a1 = __dadd_rn(a1, num[q]);
+      a2 = __dadd_rn(a2, num2[q]);
+      if (pres[q]) {
+        b1 = __dadd_rn(b1, num[q]);
+        b2 = __dadd_rn(b2, num2[q]);
+      }
+    }
+    uint64_t d[W];
+#pragma unroll
+    for (int w = 0; w < W; w++) d[w] = keys[i * W + w];
+    const double den = __dsub_rn(ptEnergy<W, LDS_TAB>(S, tab, d), e0);
+    sA = __dadd_rn(sA, __ddiv_rn(__dsub_rn(__ddiv_rn(__dmul_rn(__dmul_rn(fabs(a1), fabs(a1)), nmc), nmc - 1.0), a2),
+                                 den));
+    sB = __dadd_rn(sB, __ddiv_rn(__dsub_rn(__ddiv_rn(__dmul_rn(__dmul_rn(fabs(b1), fabs(b1)), nmc), nmc - 1.0), b2),
+                                 den));
+  }
+  const double t0 = blockSum(sA), t1 = blockSum(sB);
+  if (threadIdx.x == 0) {
+    partial[2 * blockIdx.x] = t0;
+    partial[2 * blockIdx.x + 1] = t1;
+  }
+}
 
 __global__ void kPrecondition(double* r, const double* diag, const double* e, int64_t n) {
   const double ev = e[0];
@@ -3311,49 +3383,83 @@ void launchScreen(const DevSystem& S, const uint64_t* dets, int64_t begin, int64
   HIP_CHECK(hipGetLastError());
 }
 
+void buildDenseHeatBath(const DevSystem& S, DevMem* dense, hipStream_t s) {
+  const int64_t npair = (int64_t)S.norb * (S.norb + 1) / 2, m = npair * S.norb * S.norb;
+  for (int k = 0; k < 2; k++) {
+    dense[k].reserve((size_t)m * 4, s);
+    kFillNan<<<gridFor(m), kBlock, 0, s>>>(dense[k].as<float>(), m);
+    kDenseHeatBath<<<gridFor(npair, 1), kBlock, 0, s>>>(S.hbVal[k], S.hbPair[k], S.hbStart[k], npair, S.norb,
+                                                        dense[k].as<float>());
+  }
+  HIP_CHECK(hipGetLastError());
+}
+
+int ptSlices(int64_t nsrc, int nelec) {
+  // 32,768 waves (four times what the chip holds) where the sources are
+  // fewer, in parts of at least four pairs of electrons, so that a part's own
+  // set-up (the lists of occupied and open orbitals) stays small
+  const int64_t most = 1 + std::max(1, nelec * (nelec - 1) / 2 / 4);
+  return (int)std::max<int64_t>(1, std::min<int64_t>(most, 32768 / std::max<int64_t>(nsrc, 1)));
+}
+
 void launchPtGen(const DevSystem& S, const uint64_t* dets, int64_t n, const double* ci, double eps2,
-                 const int32_t* table, uint64_t slots, uint32_t nparts, uint32_t part, int64_t* counts,
-                 const int64_t* fillStart, uint64_t* outD, double* outN, hipStream_t s) {
+                 const int32_t* table, uint64_t slots, uint32_t nparts, uint32_t part, int slices, const DevMem* dense,
+                 int64_t* counts, const int64_t* fillStart, uint64_t* outD, double* outN, hipStream_t s) {
   if (n <= 0) return;
   if (nparts == 0 || part >= nparts) throw HipError("launchPtGen: bad partition");
-  unsigned g = gridFor(n, kWaves, 1 << 16);
+  unsigned g = gridFor(n * slices, kWaves, 1 << 16);
   const PtStoch st{nullptr, nullptr, 0.0, 0.0, nullptr, nullptr};
+  const float *d0 = dense[0].as<float>(), *d1 = dense[1].as<float>();
   if (fillStart)
     DISPATCH_W(S.W, kPtGen<WW, true, false><<<g, kBlock, 0, s>>>(S, dets, n, ci, eps2, table, slots - 1, nparts, part,
-                                                                   counts, fillStart, outD, outN, st));
+                                                                   counts, fillStart, outD, outN, st, slices, d0, d1));
   else
-    DISPATCH_W(S.W, kPtGen<WW, false, false><<<g, kBlock, 0, s>>>(S, dets, n, ci, eps2, table, slots - 1, nparts,
-                                                                    part, counts, nullptr, nullptr, nullptr, st));
+    DISPATCH_W(S.W,
+               kPtGen<WW, false, false><<<g, kBlock, 0, s>>>(S, dets, n, ci, eps2, table, slots - 1, nparts, part,
+                                                              counts, nullptr, nullptr, nullptr, st, slices, d0, d1));
   HIP_CHECK(hipGetLastError());
 }
 
 void launchPtGenStoch(const DevSystem& S, const uint64_t* dets, const uint32_t* src, const double* w, int64_t nsrc,
                       const double* ci, double eps2, double eps2Large, double nmc, const int32_t* table, uint64_t slots,
-                      int64_t* counts, const int64_t* fillStart, uint64_t* outD, double* outN, double* outN2,
-                      uint8_t* outP, hipStream_t s) {
+                      int slices, const DevMem* dense, int64_t* counts, const int64_t* fillStart, uint64_t* outD,
+                      double* outN, double* outN2, uint8_t* outP, hipStream_t s) {
   if (nsrc <= 0) return;
-  unsigned g = gridFor(nsrc, kWaves, 1 << 16);
+  unsigned g = gridFor(nsrc * slices, kWaves, 1 << 16);
   const PtStoch st{src, w, eps2Large, nmc, outN2, outP};
+  const float *d0 = dense[0].as<float>(), *d1 = dense[1].as<float>();
   if (fillStart)
     DISPATCH_W(S.W, kPtGen<WW, true, true><<<g, kBlock, 0, s>>>(S, dets, nsrc, ci, eps2, table, slots - 1, 1u, 0u,
-                                                                  counts, fillStart, outD, outN, st));
+                                                                  counts, fillStart, outD, outN, st, slices, d0, d1));
   else
-    DISPATCH_W(S.W, kPtGen<WW, false, true><<<g, kBlock, 0, s>>>(S, dets, nsrc, ci, eps2, table, slots - 1, 1u, 0u,
-                                                                   counts, nullptr, nullptr, nullptr, st));
+    DISPATCH_W(S.W,
+               kPtGen<WW, false, true><<<g, kBlock, 0, s>>>(S, dets, nsrc, ci, eps2, table, slots - 1, 1u, 0u, counts,
+                                                             nullptr, nullptr, nullptr, st, slices, d0, d1));
   HIP_CHECK(hipGetLastError());
 }
 
 void launchPtStochReduce(const DevSystem& S, const uint64_t* keys, const uint32_t* idx, const double* num,
                          const double* num2, const uint8_t* pres, int64_t m, double e0, double nmc, DevMem& partial,
-                         double* out, hipStream_t s) {
+                         DevMem& counts, DevMem& starts, Workspace& ws, double* out, hipStream_t s) {
+  // over the run starts, compacted in order first, as the deterministic sum
+  const int64_t nbS = (m + kStartChunk - 1) / kStartChunk;
+  counts.reserve((size_t)(nbS + 1) * 8, s);
+  starts.reserve((size_t)m * 4, s);
+  int64_t* cnt = counts.as<int64_t>();
+  HIP_CHECK(hipMemsetAsync(cnt + nbS, 0, 8, s));
+  DISPATCH_W(S.W, kPtCountStarts<WW><<<(unsigned)nbS, kBlock, 0, s>>>(keys, m, cnt));
+  exclusiveScanI64(cnt, nbS + 1, ws, s);
+  DISPATCH_W(S.W, kPtWriteStarts<WW><<<(unsigned)nbS, kBlock, 0, s>>>(keys, m, cnt, starts.as<uint32_t>()));
   const int nb = (int)std::max<int64_t>(1, std::min<int64_t>(kPtRedBlocks, (m + kBlock - 1) / kBlock));
   partial.reserve((size_t)nb * 2 * sizeof(double));
   const size_t tb = ptTabBytes(S.norb);
   if (tb <= kPtTabMaxBytes)
-    DISPATCH_W(S.W, kPtStochReduce<WW, true><<<nb, kBlock, tb, s>>>(S, keys, idx, num, num2, pres, m, e0, nmc,
+    DISPATCH_W(S.W, kPtStochReduce<WW, true><<<nb, kBlock, tb, s>>>(S, keys, idx, num, num2, pres,
+                                                                    starts.as<uint32_t>(), cnt + nbS, m, e0, nmc,
                                                                     partial.as<double>()));
   else
-    DISPATCH_W(S.W, kPtStochReduce<WW, false><<<nb, kBlock, 0, s>>>(S, keys, idx, num, num2, pres, m, e0, nmc,
+    DISPATCH_W(S.W, kPtStochReduce<WW, false><<<nb, kBlock, 0, s>>>(S, keys, idx, num, num2, pres,
+                                                                     starts.as<uint32_t>(), cnt + nbS, m, e0, nmc,
                                                                      partial.as<double>()));
   kFinalSum<<<2, kBlock, 0, s>>>(partial.as<double>(), nb, 2, 2, out);
   HIP_CHECK(hipGetLastError());

@@ -49,3 +49,23 @@ def test_sigma_work_units(case, n, prec, tmp_path):
     x = np.random.default_rng(n).normal(size=n)
     yo = o.sigma(x)
     assert np.max(np.abs(s.hmult(x) - yo)) <= (3e-6 if prec else 1e-12) * np.max(np.abs(yo))
+
+
+@pytest.mark.parametrize("eps2", [0.0, 1e-4, 3e-2])
+@pytest.mark.parametrize("case,n", [("w1", 1), ("w1", 65), ("w2", 130)])
+def test_pt_candidates_of_few_sources(case, n, eps2, tmp_path):
+    """Few sources (cut by electron pairs), lists walked (large eps2) and open
+    orbitals enumerated (small), sums against the oracle's to 1e-11 (thousands
+    of terms of one sign in another order)."""
+    from dice_amd import shci
+    path, occ, W = _system(case, tmp_path)
+    dets = _space(path, occ, n, W)
+    s = shci.System.from_fcidump(path)
+    s.set_dets(dets)
+    c = np.random.default_rng(n).normal(size=n)
+    c /= np.linalg.norm(c)
+    e0 = s.energy(dets).min() - 2.0
+    o = OracleSystem(path)
+    got, ref = s.pt_deterministic(c, e0, eps2), o.pt_deterministic(dets, c, e0, eps2)
+    assert got[2] == ref[2]
+    np.testing.assert_allclose(got[:2], ref[:2], rtol=1e-11, atol=0)
