@@ -24,6 +24,7 @@ Engine::Engine() {}
 Engine::~Engine() {
   clearGraphs();
   if (bdHost) (void)hipHostFree(bdHost);
+  if (dvHost) (void)hipHostFree(dvHost);
   for (SigmaEvent& e : sigmaEvents) {
     (void)hipEventDestroy(e.start);
     (void)hipEventDestroy(e.stop);
@@ -1446,14 +1447,13 @@ std::vector<double> Engine::davidson(double* dX0, int nr, int maxCopies, double 
   dvS.reserve((size_t)N * maxCopies * 8);
   dvR.reserve((size_t)N * 8);
   dvScal.reserve(64 * 8);
-  dvG.reserve(512 * 8);
   dvW.reserve(32 * 8);
   dvV.reserve(256 * 8);
+  if (!dvHost) HIP_CHECK(hipHostMalloc((void**)&dvHost, 32 * 8, hipHostMallocDefault));
   double* B = dvB.as<double>();
   double* Sg = dvS.as<double>();
   double* r = dvR.as<double>();
   double* sc = dvScal.as<double>();  // [0..1] dot2, [2] norm2, [3..] residual norms
-  double* G = dvG.as<double>();
   double* Wv = dvW.as<double>();
   double* V = dvV.as<double>();
   hipStream_t s = stream;
@@ -1504,17 +1504,13 @@ std::vector<double> Engine::davidson(double* dX0, int nr, int maxCopies, double 
       sigma(col(B, i), col(Sg, i), 1, N, exactSigma);
       sigmaSize++;
     }
-    launchGram(B, bsize, Sg, bsize, N, N, G, dvPart, s);
-    launchSymmetrizeUpper(G, bsize, G + 256, s);
-    launchJacobi(G + 256, bsize, Wv, V, s);
-    launchRotate(B, bsize, N, N, V, s);
-    launchRotate(Sg, bsize, N, N, V, s);
     const int cr0 = convergedRoot;
-    // residual norms of the roots below convergedRoot, then of convergedRoot
-    for (int i = 0; i < cr0; i++) launchResidual(col(Sg, i), col(B, i), Wv + i, N, r, sc + 3 + i, dvPart, s);
-    launchResidual(col(Sg, cr0), col(B, cr0), Wv + cr0, N, r, sc + 3 + cr0, dvPart, s);
-    HIP_CHECK(hipMemcpyAsync(w.data(), Wv, bsize * 8, hipMemcpyDeviceToHost, s));
-    readScalars(hres.data(), sc + 3, cr0 + 1);
+    // eigenpairs of the subspace, the rotated vectors, and the residual norms
+    // of the roots below convergedRoot, then of convergedRoot
+    launchRayleighRitz(B, Sg, bsize, N, Wv, V, cr0, r, dvPart, dvHost, s);
+    HIP_CHECK(hipStreamSynchronize(s));
+    std::copy(dvHost, dvHost + bsize, w.begin());
+    std::copy(dvHost + 16, dvHost + 16 + cr0 + 1, hres.begin());
     const double* ePtr = Wv + cr0;  // ei = eigenvalue of the convergedRoot on entry
     for (int i = 0; i < cr0; i++) {
       if (std::sqrt(hres[i]) > tol) {
@@ -1580,21 +1576,15 @@ std::vector<double> Engine::davidson(double* dX0, int nr, int maxCopies, double 
         return eroots;
       }
     }
-    launchPrecondition(r, diag.as<double>(), ePtr, N, s);
-    for (int i = 0; i < bsize; i++) {
-      launchDot2(col(B, i), r, N, sc, dvPart, s);
-      launchOrthoStep(r, col(B, i), sc, N, s);
-    }
-    launchNorm2(r, N, sc + 2, dvPart, s);
+    const int m = bsize;  // columns the correction is made orthogonal to
     if (bsize < maxCopies) {
-      launchScaleInto(col(B, bsize), r, sc + 2, N, s);
       bsize++;
     } else {
       // restart (davidsonDirect keeps min(nroots + 3, maxCopies) vectors)
       bsize = davidsonDirectRules ? std::min(nr + 3, maxCopies) : nr + 3;
       sigmaSize = bsize - 1;
-      launchScaleInto(col(B, bsize - 1), r, sc + 2, N, s);
     }
+    launchCorrection(r, diag.as<double>(), ePtr, B, m, N, col(B, bsize - 1), dvPart, s);
   }
 }
 

@@ -113,7 +113,8 @@ struct Engine {
   void buildLowerTiled();
 
   // Davidson scratch
-  DevMem dvB, dvS, dvR, dvScal, dvPart, dvG, dvW, dvV, dvX;
+  DevMem dvB, dvS, dvR, dvScal, dvPart, dvW, dvV;
+  double* dvHost = nullptr;  // pinned: Ritz values and residual norms
   // the reference's direct mode (`directdavidson`): no stored H, sigma from
   // the string tables (HmultDirect), and davidsonDirect's restart size,
   // iteration cap and progress lines (printed to davidsonPrint when set)

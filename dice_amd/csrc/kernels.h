@@ -315,11 +315,20 @@ void launchSymRowBound(const TiledHam& T, const uint32_t* pos, const uint32_t* b
                        unsigned long long* bound, hipStream_t s);
 
 // --- Davidson vector kernels ----------------------------------------------------------
-// G[i*mb + j] = A[:,i] . B[:,j] for i < ma, j < mb (columns of length n, ld)
+// Rayleigh-Ritz of the single-vector Davidson: the Gram matrix B^T S of m
+// columns (of length n, one after the other; its upper triangle mirrored), its
+// eigenvalues w (ascending) and eigenvectors V (cyclic Jacobi), B and S
+// rotated by V, r = the residual S_last - w_last B_last; host (32 values the
+// device can write): w, then from 16 on ||S_i - w_i B_i||^2 for i <= last
+void launchRayleighRitz(double* B, double* S, int m, int64_t n, double* w, double* V, int last, double* r,
+                        DevMem& partial, double* host, hipStream_t s);
+// r = r / (e - diag) with the 1e-12 guard, orthogonalised against B's m
+// columns one after the other, and normalised into dst
+void launchCorrection(double* r, const double* diag, const double* e, const double* B, int m, int64_t n, double* dst,
+                      DevMem& partial, hipStream_t s);
+// G[0] = A . B (one column each)
 void launchGram(const double* A, int ma, const double* B, int mb, int64_t n, int64_t ld, double* G,
                 DevMem& partial, hipStream_t s);
-// X[:, :m] = X[:, :m] * V (V row-major m x m on device)
-void launchRotate(double* X, int m, int64_t n, int64_t ld, const double* V, hipStream_t s);
 // out[i*cols + j] = C[i*ldc + j] for i < rows, j < cols (small matrices)
 void launchSubMatrix(const double* C, int ldc, int rows, int cols, double* out, hipStream_t s);
 // G[i*mb + j] = A[:,i] . B[:,j] for ma, mb <= 64 (8 x 8 tiles; fixed-order sums)
@@ -346,11 +355,9 @@ void launchScaleInto(double* dst, const double* src, const double* nrm2, int64_t
 void launchAxpy(double* x, const double* y, double alpha, int64_t n, hipStream_t s);
 // A[i*m+j] = G[min(i,j)*m + max(i,j)]  (upper triangle mirrored)
 void launchSymmetrizeUpper(const double* G, int m, double* A, hipStream_t s);
-// symmetric eigen-decomposition of the m x m matrix (row-major) by cyclic
-// Jacobi, eigenvalues ascending in w, eigenvectors in the columns of V
-void launchJacobi(const double* A, int m, double* w, double* V, hipStream_t s);
-// the same with the rotations of a sweep in round-robin order (disjoint pairs
-// at once): eigenpairs equal to rounding, fewer barriers (block Davidson)
+// symmetric eigen-decomposition of the m x m matrix (row-major) by Jacobi
+// sweeps with the rotations in round-robin order (disjoint pairs at once),
+// eigenvalues ascending in w, eigenvectors in the columns of V (block Davidson)
 void launchJacobiRR(const double* A, int m, double* w, double* V, hipStream_t s);
 
 }  // namespace shci

@@ -2761,22 +2761,6 @@ __global__ void __launch_bounds__(kBlock) kGramFinal(const double* partial, int 
   }
 }
 
-__global__ void kRotate(double* X, int m, int64_t n, int64_t ld, const double* V) {
-  __shared__ double sV[16 * 16];
-  for (int q = threadIdx.x; q < m * m; q += blockDim.x) sV[q] = V[q];
-  __syncthreads();
-  for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x) {
-    double xin[16], xo[16];
-    for (int l = 0; l < m; l++) xin[l] = X[l * ld + k];
-    for (int j = 0; j < m; j++) {
-      double s = 0.0;
-      for (int l = 0; l < m; l++) s = fma(xin[l], sV[l * m + j], s);
-      xo[j] = s;
-    }
-    for (int j = 0; j < m; j++) X[j * ld + k] = xo[j];
-  }
-}
-
 // Gram tiles: blockIdx.y = tile (ta, tb) of 8 x 8 entries
 __global__ void __launch_bounds__(kBlock) kGramTile(const double* A, int ma, const double* B, int mb, int64_t n,
                                                     int64_t ld, double* partial) {
@@ -3119,70 +3103,67 @@ __global__ void kSymUpper(const double* G, int m, double* A) {
 // Cyclic Jacobi for m <= kJacobiMax on one wavefront with the matrices in
 // LDS: rotations are applied in the sequential (p, q) order, lane k updating
 // element k of the two rows / columns, so every element sees the same
-// operations in the same order as a one-thread sweep.
+// operations in the same order as a one-thread sweep.  It is one chain of
+// dependent operations (a rotation's angle, then its rows and columns), so
+// what counts is the LDS round trips in it: two per rotation beside the read
+// of the pivot.
 constexpr int kJacobiMax = 32;
 
-__global__ void __launch_bounds__(64) kJacobi(const double* A, int m, double* w, double* V) {
-  __shared__ double a[kJacobiMax * kJacobiMax], v[kJacobiMax * kJacobiMax];
-  __shared__ double sOff;
-  __shared__ int order[kJacobiMax];
-  const int lane = threadIdx.x;
-  for (int q = lane; q < m * m; q += 64) {
-    a[q] = A[q];
-    v[q] = 0.0;
-  }
-  __syncthreads();
-  if (lane < m) v[lane * m + lane] = 1.0;
-  __syncthreads();
+// the wave's LDS writes are seen by its lanes' later reads
+__device__ __forceinline__ void waveSync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// a: the matrix (LDS, overwritten), v, order: LDS scratch; called by the 64
+// lanes of one wave
+__device__ void jacobiWave(double* a, double* v, int* order, int m, double* w, double* V) {
+  const int lane = __lane_id();
+  for (int q = lane; q < m * m; q += 64) v[q] = q / m == q % m ? 1.0 : 0.0;
+  waveSync();
   for (int sweep = 0; sweep < 100; sweep++) {
-    if (lane == 0) {
-      double off = 0.0;
-      for (int p = 0; p < m; p++)
-        for (int q = p + 1; q < m; q++) off += fabs(a[p * m + q]);
-      sOff = off;
-    }
-    __syncthreads();
-    if (sOff == 0.0) break;
+    bool off = false;  // any element above the diagonal that is not zero
+    for (int t = lane; t < m * m; t += 64) off |= t % m > t / m && a[t] != 0.0;
+    if (__ballot(off) == 0ull) break;
     for (int p = 0; p < m; p++)
       for (int q = p + 1; q < m; q++) {
         const double apq = a[p * m + q], app = a[p * m + p], aqq = a[q * m + q];
         const double g = 100.0 * fabs(apq);
         if (sweep > 3 && fabs(app) + g == fabs(app) && fabs(aqq) + g == fabs(aqq)) {
-          __syncthreads();
+          waveSync();
           if (lane == 0) {
             a[p * m + q] = 0.0;
             a[q * m + p] = 0.0;
           }
-          __syncthreads();
+          waveSync();
           continue;
         }
         if (apq == 0.0) continue;
+        double akp = 0.0, akq = 0.0, vkp = 0.0, vkq = 0.0;
+        if (lane < m) {
+          akp = a[lane * m + p];
+          akq = a[lane * m + q];
+          vkp = v[lane * m + p];
+          vkq = v[lane * m + q];
+        }
         const double theta = (aqq - app) / (2.0 * apq);
         const double t = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
         const double c = 1.0 / sqrt(t * t + 1.0), sn = t * c;
-        __syncthreads();
+        waveSync();
         if (lane < m) {
-          const double akp = a[lane * m + p], akq = a[lane * m + q];
           a[lane * m + p] = c * akp - sn * akq;
           a[lane * m + q] = sn * akp + c * akq;
-        }
-        __syncthreads();
-        if (lane < m) {
-          const double apk = a[p * m + lane], aqk = a[q * m + lane];
-          a[p * m + lane] = c * apk - sn * aqk;
-          a[q * m + lane] = sn * apk + c * aqk;
-          const double vkp = v[lane * m + p], vkq = v[lane * m + q];
           v[lane * m + p] = c * vkp - sn * vkq;
           v[lane * m + q] = sn * vkp + c * vkq;
         }
-        __syncthreads();
-        if (lane == 0) {
-          a[p * m + q] = 0.0;
-          a[q * m + p] = 0.0;
+        waveSync();
+        if (lane < m) {
+          const double apk = a[p * m + lane], aqk = a[q * m + lane];
+          a[p * m + lane] = lane == q ? 0.0 : c * apk - sn * aqk;
+          a[q * m + lane] = lane == p ? 0.0 : sn * apk + c * aqk;
         }
-        __syncthreads();
+        waveSync();
       }
-    __syncthreads();
   }
   if (lane == 0) {
     for (int i = 0; i < m; i++) order[i] = i;
@@ -3196,7 +3177,7 @@ __global__ void __launch_bounds__(64) kJacobi(const double* A, int m, double* w,
       order[j] = o;
     }
   }
-  __syncthreads();
+  waveSync();
   if (lane < m) w[lane] = a[order[lane] * m + order[lane]];
   for (int q = lane; q < m * m; q += 64) {
     const int k = q / m, j = q % m;
@@ -3204,11 +3185,264 @@ __global__ void __launch_bounds__(64) kJacobi(const double* A, int m, double* w,
   }
 }
 
+// ---- one step of the single-vector Davidson, in few launches --------------
+//
+// On small spaces its time was the launches: three for every dot product and
+// step of the orthogonalisation, two for each norm, one for each rotation.
+// Here a kernel that needs a sum over the vector ends the reduction of the
+// previous kernel itself, every workgroup by itself and all in the same fixed
+// order, and leaves its own partial sums for the next one.  Every element
+// and every sum takes the operations of separate kernels for the Gram matrix,
+// its eigenpairs, the rotation, the residual, the preconditioner, each dot
+// product, each orthogonalisation step and the norms, in their order: the
+// same bits.  With m columns m + 7 launches in place of 3 m + 13 and more, and
+// the scalars the host decides on come through memory it can read.  The
+// two-root solve on 57,963 determinants of 40 orbitals (184 iterations) 52 ->
+// 30 ms, the whole step of an 8-orbital molecule (86 iterations) 20 -> 16.
+
+// v summed over the wave as the xor tree 32, 16, 8, 4, 2, 1: the last four
+// steps rotate within rows of 16 lanes (a step's value repeats with its
+// distance, so the rotation brings what the xor would), without LDS
+template <int CTRL>
+__device__ __forceinline__ double dppAdd(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+  return v + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double waveSumXor(double v) {
+  v += __shfl_xor(v, 32, 64);
+  v += __shfl_xor(v, 16, 64);
+  v = dppAdd<0x128>(v);  // row_ror:8
+  v = dppAdd<0x124>(v);
+  v = dppAdd<0x122>(v);
+  return dppAdd<0x121>(v);
+}
+
+// the workgroup's sums of v[NV], as blockSum; every thread gets them
+template <int NV>
+__device__ __forceinline__ void blockSums(double (&v)[NV], double* red) {
+  const int wave = threadIdx.x >> 6, lane = __lane_id();
+#pragma unroll
+  for (int q = 0; q < NV; q++) {
+    const double t = waveSumXor(v[q]);
+    if (lane == 0) red[q * kWaves + wave] = t;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < NV; q++) {
+    double t = 0.0;
+    for (int w = 0; w < kWaves; w++) t += red[q * kWaves + w];
+    v[q] = t;
+  }
+  __syncthreads();
+}
+
+// the sums kFinalSum forms of nb partials of NV values
+template <int NV>
+__device__ __forceinline__ void finalSums(const double* partial, int nb, double (&v)[NV], double* red) {
+#pragma unroll
+  for (int q = 0; q < NV; q++) {
+    v[q] = 0.0;
+    for (int b = threadIdx.x; b < nb; b += kBlock) v[q] += partial[(int64_t)b * NV + q];
+  }
+  blockSums<NV>(v, red);
+}
+
+// partial Gram entries B_i . S_j, i <= j, of exactly M columns
+template <int M>
+__global__ void __launch_bounds__(kBlock) kGramUpper(const double* __restrict__ B, const double* __restrict__ S,
+                                                     int64_t n, int64_t ld, double* __restrict__ partial) {
+  constexpr int Q = M * (M + 1) / 2;
+  __shared__ double red[kWaves][Q];
+  double acc[Q];
+#pragma unroll
+  for (int q = 0; q < Q; q++) acc[q] = 0.0;
+  for (int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x; k < n; k += (int64_t)gridDim.x * kBlock) {
+    double a[M], b[M];
+#pragma unroll
+    for (int i = 0; i < M; i++) {
+      a[i] = B[i * ld + k];
+      b[i] = S[i * ld + k];
+    }
+    int q = 0;
+#pragma unroll
+    for (int i = 0; i < M; i++)
+#pragma unroll
+      for (int j = i; j < M; j++, q++) acc[q] = fma(a[i], b[j], acc[q]);
+  }
+  const int wave = threadIdx.x >> 6, lane = __lane_id();
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    const double t = waveSumXor(acc[q]);
+    if (lane == 0) red[wave][q] = t;
+  }
+  __syncthreads();
+  for (int q = threadIdx.x; q < Q; q += kBlock) {
+    double v = 0.0;
+    for (int w = 0; w < kWaves; w++) v += red[w][q];
+    partial[(int64_t)blockIdx.x * Q + q] = v;
+  }
+}
+
+// the Gram matrix from those partials (a wave per entry: the four wave sums
+// of kGramFinal one after the other) and its eigenpairs; one workgroup
+constexpr int kGramThreads = 1024;
+__global__ void __launch_bounds__(kGramThreads) kGramJacobi(const double* __restrict__ partial, int nb, int m,
+                                                            double* w, double* V) {
+  __shared__ double a[kJacobiMax * kJacobiMax], v[kJacobiMax * kJacobiMax];
+  __shared__ int order[kJacobiMax];
+  const int wave = threadIdx.x >> 6, lane = __lane_id(), Q = m * (m + 1) / 2;
+  for (int q = wave; q < Q; q += kGramThreads / 64) {
+    double t = 0.0;
+    for (int c = 0; c < kWaves; c++) {
+      double u = 0.0;
+      for (int b = c * 64 + lane; b < nb; b += kBlock) u += partial[(int64_t)b * Q + q];
+      t += waveSumXor(u);
+    }
+    int i = 0, r = q;
+    while (r >= m - i) {
+      r -= m - i;
+      i++;
+    }
+    if (lane == 0) {
+      a[i * m + i + r] = t;
+      a[(i + r) * m + i] = t;
+    }
+  }
+  __syncthreads();
+  if (wave == 0) jacobiWave(a, v, order, m, w, V);
+}
+
+// B and S rotated by V (m x m), the residuals S_i - w_i B_i of the columns
+// i <= last (r: the last one), and the partial sums of their squares
+constexpr int kResMax = 12;
+__global__ void __launch_bounds__(kBlock) kRotateResidual(double* B, double* S, int m, int64_t n, int64_t ld,
+                                                          const double* V, const double* w, int last, double* r,
+                                                          double* partial) {
+  __shared__ double sV[16 * 16];
+  __shared__ double red[kWaves];
+  for (int q = threadIdx.x; q < m * m; q += kBlock) sV[q] = V[q];
+  __syncthreads();
+  double acc[kResMax];
+#pragma unroll
+  for (int i = 0; i < kResMax; i++) acc[i] = 0.0;
+  for (int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x; k < n; k += (int64_t)gridDim.x * kBlock) {
+    double bi[16], si[16];
+#pragma unroll
+    for (int l = 0; l < 16; l++)
+      if (l < m) {
+        bi[l] = B[l * ld + k];
+        si[l] = S[l * ld + k];
+      }
+#pragma unroll
+    for (int j = 0; j < 16; j++) {
+      if (j >= m) break;
+      double bo = 0.0, so = 0.0;
+#pragma unroll
+      for (int l = 0; l < 16; l++)
+        if (l < m) {
+          bo = fma(bi[l], sV[l * m + j], bo);
+          so = fma(si[l], sV[l * m + j], so);
+        }
+      B[j * ld + k] = bo;
+      S[j * ld + k] = so;
+      if (j < kResMax && j <= last) {
+        const double d = so - w[j] * bo;
+        if (j == last) r[k] = d;
+        acc[j] = fma(d, d, acc[j]);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kResMax; j++) {
+    if (j > last) break;
+    double t[1] = {acc[j]};
+    blockSums<1>(t, red);
+    if (threadIdx.x == 0) partial[(int64_t)blockIdx.x * (last + 1) + j] = t[0];
+  }
+}
+
+// the residuals' sums, with the eigenvalues, to host memory: w (16), sums
+__global__ void __launch_bounds__(kBlock) kResidualSums(const double* partial, int nb, int count, const double* w,
+                                                        int m, double* host) {
+  __shared__ double red[kWaves];
+  for (int q = 0; q < count; q++) {
+    double v[1] = {0.0};
+    for (int b = threadIdx.x; b < nb; b += kBlock) v[0] += partial[(int64_t)b * count + q];
+    blockSums<1>(v, red);
+    if (threadIdx.x == 0) host[16 + q] = v[0];
+  }
+  if ((int)threadIdx.x < m) host[threadIdx.x] = w[threadIdx.x];
+}
+
+// r /= e - diag (kPrecondition) and the partials of b . r and b . b
+__global__ void __launch_bounds__(kBlock) kPreconditionDot(double* r, const double* __restrict__ diag, const double* e,
+                                                           const double* __restrict__ b, int64_t n, double* out) {
+  __shared__ double red[2 * kWaves];
+  const double ev = e[0];
+  double v[2] = {0.0, 0.0};
+  for (int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x; k < n; k += (int64_t)gridDim.x * kBlock) {
+    const double den = ev - diag[k];
+    const double x = fabs(den) > 1e-12 ? r[k] / den : r[k] / (den - 1.e-12);
+    r[k] = x;
+    const double bv = b[k];
+    v[0] = fma(bv, x, v[0]);
+    v[1] = fma(bv, bv, v[1]);
+  }
+  blockSums<2>(v, red);
+  if (threadIdx.x == 0) {
+    out[2 * blockIdx.x] = v[0];
+    out[2 * blockIdx.x + 1] = v[1];
+  }
+}
+
+// r -= (b . r) b / (b . b) with the sums of `in`, then the partials of next . r
+// and next . next, or (next null) of r . r
+__global__ void __launch_bounds__(kBlock) kOrthoDot(double* r, const double* __restrict__ b,
+                                                    const double* __restrict__ next, int64_t n, const double* in,
+                                                    double* out) {
+  __shared__ double red[2 * kWaves];
+  double s[2];
+  finalSums<2>(in, (int)gridDim.x, s, red);
+  double v[2] = {0.0, 0.0};
+  for (int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x; k < n; k += (int64_t)gridDim.x * kBlock) {
+    const double x = r[k] - s[0] * b[k] / s[1];
+    r[k] = x;
+    if (next) {
+      const double bv = next[k];
+      v[0] = fma(bv, x, v[0]);
+      v[1] = fma(bv, bv, v[1]);
+    } else {
+      v[0] = fma(x, x, v[0]);
+    }
+  }
+  blockSums<2>(v, red);
+  if (threadIdx.x == 0) {
+    if (next) {
+      out[2 * blockIdx.x] = v[0];
+      out[2 * blockIdx.x + 1] = v[1];
+    } else {
+      out[blockIdx.x] = v[0];
+    }
+  }
+}
+
+// dst = r / sqrt(sum of in)
+__global__ void __launch_bounds__(kBlock) kScaleSum(double* dst, const double* __restrict__ r, int64_t n,
+                                                    const double* in) {
+  __shared__ double red[kWaves];
+  double s[1];
+  finalSums<1>(in, (int)gridDim.x, s, red);
+  const double nr = sqrt(s[0]);
+  for (int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x; k < n; k += (int64_t)gridDim.x * kBlock)
+    dst[k] = r[k] / nr;
+}
+
 // The same eigenproblem with the rotations of a sweep in round-robin
 // (tournament) order: the m'/2 disjoint pairs of a step (m' = m rounded up
 // to even) are rotated at once, m'-1 steps per sweep, so a sweep needs
 // m'-1 rounds of barriers instead of m(m-1)/2.  Another rotation order than
-// kJacobi's, so the eigenpairs agree with it to rounding, not bit for bit;
+// jacobiWave's, so the eigenpairs agree with it to rounding, not bit for bit;
 // used by the block Davidson.
 __global__ void __launch_bounds__(64) kJacobiRR(const double* A, int m, double* w, double* V) {
   __shared__ double a[kJacobiMax * kJacobiMax], v[kJacobiMax * kJacobiMax];
@@ -4314,18 +4548,6 @@ void launchGram(const double* A, int ma, const double* B, int mb, int64_t n, int
     partial.reserve((size_t)nbb * 1 * sizeof(double));
     kGramPartial<1, 1><<<nbb, kBlock, 0, s>>>(A, B, ma, mb, n, ld, partial.as<double>());
     kGramFinal<<<ma * mb, kBlock, 0, s>>>(partial.as<double>(), nbb, 1, 1, ma, mb, G);
-  } else if (ma <= 1 && mb <= 8) {
-    partial.reserve((size_t)nbb * 8 * sizeof(double));
-    kGramPartial<1, 8><<<nbb, kBlock, 0, s>>>(A, B, ma, mb, n, ld, partial.as<double>());
-    kGramFinal<<<ma * mb, kBlock, 0, s>>>(partial.as<double>(), nbb, 1, 8, ma, mb, G);
-  } else if (ma <= 8 && mb <= 8) {
-    partial.reserve((size_t)nbb * 64 * sizeof(double));
-    kGramPartial<8, 8><<<nbb, kBlock, 0, s>>>(A, B, ma, mb, n, ld, partial.as<double>());
-    kGramFinal<<<ma * mb, kBlock, 0, s>>>(partial.as<double>(), nbb, 8, 8, ma, mb, G);
-  } else if (ma <= 12 && mb <= 12) {
-    partial.reserve((size_t)nbb * 144 * sizeof(double));
-    kGramPartial<12, 12><<<nbb, kBlock, 0, s>>>(A, B, ma, mb, n, ld, partial.as<double>());
-    kGramFinal<<<ma * mb, kBlock, 0, s>>>(partial.as<double>(), nbb, 12, 12, ma, mb, G);
   } else {
     throw HipError("launchGram: subspace too large");
   }
@@ -4359,12 +4581,6 @@ __global__ void kSubMatrix(const double* C, int ldc, int rows, int cols, double*
 void launchSubMatrix(const double* C, int ldc, int rows, int cols, double* out, hipStream_t s) {
   if (rows <= 0 || cols <= 0) return;
   kSubMatrix<<<1, kBlock, 0, s>>>(C, ldc, rows, cols, out);
-  HIP_CHECK(hipGetLastError());
-}
-
-void launchRotate(double* X, int m, int64_t n, int64_t ld, const double* V, hipStream_t s) {
-  if (m > 16) throw HipError("launchRotate: subspace too large");
-  kRotate<<<gridFor(n, kBlock, 4096), kBlock, 0, s>>>(X, m, n, ld, V);
   HIP_CHECK(hipGetLastError());
 }
 
@@ -4424,9 +4640,49 @@ void launchJacobiRR(const double* A, int m, double* w, double* V, hipStream_t s)
   HIP_CHECK(hipGetLastError());
 }
 
-void launchJacobi(const double* A, int m, double* w, double* V, hipStream_t s) {
-  if (m > kJacobiMax) throw HipError("launchJacobi: subspace too large");
-  kJacobi<<<1, 64, 0, s>>>(A, m, w, V);
+static int redGrid(int64_t n) {
+  return (int)std::max<int64_t>(1, std::min<int64_t>(kRedBlocks, (n + kBlock - 1) / kBlock));
+}
+
+void launchRayleighRitz(double* B, double* S, int m, int64_t n, double* w, double* V, int last, double* r,
+                        DevMem& partial, double* host, hipStream_t s) {
+  if (m < 1 || m > 12 || last < 0 || last >= m || last >= kResMax) throw HipError("launchRayleighRitz: bad subspace");
+  const int nb = redGrid(n);
+  partial.reserve((size_t)nb * 78 * sizeof(double));
+  double* p = partial.as<double>();
+#define GRAM_CASE(M) \
+  case M: kGramUpper<M><<<nb, kBlock, 0, s>>>(B, S, n, n, p); break
+  switch (m) {
+    GRAM_CASE(1);
+    GRAM_CASE(2);
+    GRAM_CASE(3);
+    GRAM_CASE(4);
+    GRAM_CASE(5);
+    GRAM_CASE(6);
+    GRAM_CASE(7);
+    GRAM_CASE(8);
+    GRAM_CASE(9);
+    GRAM_CASE(10);
+    GRAM_CASE(11);
+    GRAM_CASE(12);
+  }
+#undef GRAM_CASE
+  kGramJacobi<<<1, kGramThreads, 0, s>>>(p, nb, m, w, V);
+  kRotateResidual<<<nb, kBlock, 0, s>>>(B, S, m, n, n, V, w, last, r, p);
+  kResidualSums<<<1, kBlock, 0, s>>>(p, nb, last + 1, w, m, host);
+  HIP_CHECK(hipGetLastError());
+}
+
+void launchCorrection(double* r, const double* diag, const double* e, const double* B, int m, int64_t n, double* dst,
+                      DevMem& partial, hipStream_t s) {
+  const int nb = redGrid(n);
+  partial.reserve((size_t)nb * 4 * sizeof(double));
+  double* p[2] = {partial.as<double>(), partial.as<double>() + 2 * nb};
+  kPreconditionDot<<<nb, kBlock, 0, s>>>(r, diag, e, B, n, p[0]);
+  for (int i = 0; i < m; i++)
+    kOrthoDot<<<nb, kBlock, 0, s>>>(r, B + (int64_t)i * n, i + 1 < m ? B + (int64_t)(i + 1) * n : nullptr, n, p[i & 1],
+                                    p[(i + 1) & 1]);
+  kScaleSum<<<nb, kBlock, 0, s>>>(dst, r, n, p[m & 1]);
   HIP_CHECK(hipGetLastError());
 }
 

@@ -69,3 +69,34 @@ def test_pt_candidates_of_few_sources(case, n, eps2, tmp_path):
     got, ref = s.pt_deterministic(c, e0, eps2), o.pt_deterministic(dets, c, e0, eps2)
     assert got[2] == ref[2]
     np.testing.assert_allclose(got[:2], ref[:2], rtol=1e-11, atol=0)
+
+
+@pytest.mark.parametrize("n", [3, 8, 257, 1500])
+@pytest.mark.parametrize("roots", [1, 2, 9])
+def test_davidson_subspaces(n, roots, tmp_path):
+    """Every subspace size, up to 12 columns and up to the whole space, and
+    vectors shorter than a workgroup: roots against the dense eigenvalues of
+    the GPU's own rows to 1e-8 (a residual below 1e-5, so the square of it
+    over the gaps)."""
+    from dice_amd import shci
+    if roots + 3 > 12 or roots > n:
+        pytest.skip("more roots than determinants")
+    path, occ, W = _system("w1", tmp_path)
+    dets = _space(path, occ, n, W)
+    s = shci.System.from_fcidump(path)
+    s.set_dets(dets)
+    rp, cols, vals = s.hamiltonian_rows()
+    H = np.zeros((n, n))
+    for i in range(n):
+        H[i, cols[rp[i]:rp[i + 1]]] = vals[rp[i]:rp[i + 1]]
+    H = np.tril(H) + np.tril(H, -1).T
+    x0 = np.random.default_rng(n).normal(size=(n, roots))
+    x0[:roots] += 5.0 * np.eye(roots)
+    e, x, _ = s.davidson(x0, max_copies=max(roots + 3, 4), tol=1e-5)
+    resid = np.linalg.norm(H @ x - x * e, axis=0)
+    assert np.max(resid) < 2e-5
+    if n <= 8:
+        np.testing.assert_allclose(e, np.linalg.eigvalsh(H)[:roots], rtol=0, atol=1e-8)
+    else:
+        ev = np.linalg.eigvalsh(H)
+        assert all(np.min(np.abs(ev - v)) < 1e-8 for v in e)
