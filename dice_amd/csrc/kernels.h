@@ -139,7 +139,9 @@ struct StringTables {
   DevMem aSinglesStart, aSingles;  // alpha strings one excitation apart (int64 / u32)
   DevMem bSinglesStart, bSingles;  // beta strings one excitation apart (int64 / u32)
   DevMem aSortB, aSortDet;         // alpha-major groups with members by beta string: beta (u64), det (u32)
-  DevMem key, val;              // scratch
+  DevMem bmSlot, bm;            // bitmaps of the large alpha groups over the beta strings: slot per group, words
+  int64_t bmWords = 0;          // words of a bitmap
+  DevMem key, val, bmFlag;      // scratch
 };
 void buildStringTables(const DevSystem& S, const uint64_t* dets, int64_t n, StringTables& T, Workspace& ws,
                        hipStream_t s);

@@ -100,3 +100,33 @@ def test_davidson_subspaces(n, roots, tmp_path):
     else:
         ev = np.linalg.eigvalsh(H)
         assert all(np.min(np.abs(ev - v)) < 1e-8 for v in e)
+
+
+@pytest.mark.parametrize("half", [True, False])
+@pytest.mark.parametrize("size", [63, 511, 512, 700])
+def test_rows_of_groups_with_and_without_bitmap(size, half, tmp_path, monkeypatch):
+    """Three alpha strings times `size` beta strings, below and above the
+    group size from which beta singles are looked up in a bitmap, in random
+    order: rows equal the oracle's."""
+    import itertools
+    from dice_amd import shci, synth
+    path = str(tmp_path / "FCIDUMP")
+    synth.write_molecular_fcidump(path, 7, 16, 1, 4, 24)
+    rng = np.random.default_rng(size)
+    beta = list(itertools.combinations(range(16), 4))
+    beta = [beta[i] for i in rng.permutation(len(beta))[:size]]
+    dets = np.array([(1 << (2 * a)) | sum(1 << (2 * x + 1) for x in b) for a in range(3) for b in beta],
+                    dtype=np.int64).reshape(-1, 1)
+    dets = dets[rng.permutation(len(dets))]
+    monkeypatch.setenv("SHCI_STORAGE", "half" if half else "full")
+    s, o = shci.System.from_fcidump(path), OracleSystem(path)
+    s.set_dets(dets)
+    rp, cols, vals = s.hamiltonian_rows()
+    o.csr_append(dets)
+    orp, ocols, ovals = o.csr()
+    np.testing.assert_array_equal(rp, orp)
+    for i in range(len(dets)):
+        a, b = rp[i], rp[i + 1]
+        order = np.argsort(ocols[a + 1:b], kind="stable")
+        np.testing.assert_array_equal(cols[a + 1:b], ocols[a + 1:b][order])
+        np.testing.assert_array_equal(vals[a + 1:b], ovals[a + 1:b][order])
