@@ -266,7 +266,8 @@ struct TiledHam {
   int64_t n = -1, blocks = 0, segments = 0, nnz = 0, instructions = 0;
   bool f32 = false, split = false, hasLo = false;
   // lo: the FP32 values' remainders (lo = fp32(v - hi)), when built with them
-  DevMem segBase, segTile, segCnt, segStart, segInst, segTotal, fill, blockE, blockI, idx, vals, lo, inst;
+  DevMem segBase, segTile, segCnt, segStart, segInst, segTotal, fill, blockE, blockI, idx, vals, lo, inst,
+      tileBits;
   // the half-storage sigma's order: the segments by (super block, tile, row
   // block), its instructions (symInst), tile groups and work units
   DevMem order, blockOf, bigI, smallI, lead, groups, symInst, unitStart, units;

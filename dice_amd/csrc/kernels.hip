@@ -2002,28 +2002,8 @@ __device__ __forceinline__ T blockInclusiveScan(T v, T* total) {
   return v + before;
 }
 
-// marks the tiles the block's entries touch in bits[nwords] (LDS, cleared
-// here); with pre given, pre[k] = set bits before word k; returns the
-// number of touched tiles
-__device__ int tileBitmap(const int64_t* __restrict__ rowPtr, const int32_t* __restrict__ cols,
-                          const uint32_t* __restrict__ perm, const uint32_t* __restrict__ pos,
-                          const uint32_t* __restrict__ bIdx, const uint32_t* __restrict__ bPos, int64_t n,
-                          int64_t b, int nwords, uint32_t* bits, uint32_t* pre) {
-  const int wave = threadIdx.x >> 6, lane = __lane_id();
-  for (int k = threadIdx.x; k < nwords; k += kBlock) bits[k] = 0u;
-  __syncthreads();
-  const int64_t m0 = b * kTileRows;
-  const int rows = (int)(n - m0 < kTileRows ? n - m0 : kTileRows);
-  for (int r = wave; r < rows; r += kWaves) {
-    const int64_t I = perm ? (int64_t)perm[m0 + r] : m0 + r;
-    const int64_t e0 = rowPtr[I], e1 = rowPtr[I + 1];
-    const uint32_t bi = bIdx ? bIdx[I] : 0u;
-    for (int64_t p = e0 + lane; p < e1; p += 64) {
-      const uint32_t t = tileMapCol(cols[p], bi, pos, bIdx, bPos, n) >> kTileLog;
-      atomicOr(&bits[t >> 5], 1u << (t & 31));
-    }
-  }
-  __syncthreads();
+// pre[k] = set bits before word k of bits[nwords]; returns the set bits
+__device__ int tilePrefix(int nwords, const uint32_t* bits, uint32_t* pre) {
   const int per = (nwords + kBlock - 1) / kBlock;
   const int k0 = threadIdx.x * per, k1 = k0 + per < nwords ? k0 + per : nwords;
   int local = 0;
@@ -2043,12 +2023,37 @@ __device__ __forceinline__ uint32_t tileRank(const uint32_t* bits, const uint32_
   return pre[t >> 5] + __popc(bits[t >> 5] & ((1u << (t & 31)) - 1u));
 }
 
-// pass 1: touched tiles per block (segCount[b])
+// The build's passes wait for the row entries that they read: the tiles of a
+// block are found once (kTileMark) and its bitmap kept, 4 nwords bytes a block,
+// where each pass walked the block's entries for it; and the LDS follows the
+// number of tiles (bits and pre, nwords words each), where room for the largest
+// number allowed three workgroups per CU. 400,009 determinants, 24 orbitals:
+// kTileCount 1.96 -> 1.08 ms, kTileFill 4.15 -> 3.23.
+
+// pass 1: the tiles each block's entries touch (a bitmap per block, kept for
+// the other passes) and their number (segCount[b])
 __global__ void __launch_bounds__(kBlock) kTileMark(const int64_t* rowPtr, const int32_t* cols, const uint32_t* perm,
                                                     const uint32_t* pos, const uint32_t* bIdx, const uint32_t* bPos,
-                                                    int64_t n, int nwords, int64_t* segCount) {
-  __shared__ uint32_t bits[kTileMaxWords];
-  const int total = tileBitmap(rowPtr, cols, perm, pos, bIdx, bPos, n, blockIdx.x, nwords, bits, nullptr);
+                                                    int64_t n, int nwords, int64_t* segCount, uint32_t* blockBits) {
+  extern __shared__ uint32_t bits[];
+  const int wave = threadIdx.x >> 6, lane = __lane_id();
+  for (int k = threadIdx.x; k < nwords; k += kBlock) bits[k] = 0u;
+  __syncthreads();
+  const int64_t m0 = (int64_t)blockIdx.x * kTileRows;
+  const int rows = (int)(n - m0 < kTileRows ? n - m0 : kTileRows);
+  for (int r = wave; r < rows; r += kWaves) {
+    const int64_t I = perm ? (int64_t)perm[m0 + r] : m0 + r;
+    const int64_t e0 = rowPtr[I], e1 = rowPtr[I + 1];
+    const uint32_t bi = bIdx ? bIdx[I] : 0u;
+    for (int64_t p = e0 + lane; p < e1; p += 64) {
+      const uint32_t t = tileMapCol(cols[p], bi, pos, bIdx, bPos, n) >> kTileLog;
+      const uint32_t bit = 1u << (t & 31);
+      if (!(bits[t >> 5] & bit)) atomicOr(&bits[t >> 5], bit);
+    }
+  }
+  __syncthreads();
+  for (int k = threadIdx.x; k < nwords; k += kBlock) blockBits[(int64_t)blockIdx.x * nwords + k] = bits[k];
+  const int total = tilePrefix(nwords, bits, nullptr);
   if (threadIdx.x == 0) segCount[blockIdx.x] = total;
 }
 
@@ -2058,15 +2063,17 @@ __global__ void __launch_bounds__(kBlock) kTileMark(const int64_t* rowPtr, const
 // the segment; per block its entries and instructions
 __global__ void __launch_bounds__(kBlock) kTileCount(const int64_t* rowPtr, const int32_t* cols, const uint32_t* perm,
                                                      const uint32_t* pos, const uint32_t* bIdx, const uint32_t* bPos,
-                                                     int64_t n, int nwords, const int64_t* segBase, uint32_t* segTile,
-                                                     uint32_t* segCnt, uint32_t* segStart, uint32_t* segInst,
-                                                     uint32_t* segTotal, uint32_t* fill, int64_t* blockE,
-                                                     int64_t* blockI) {
-  __shared__ uint32_t bits[kTileMaxWords];
-  __shared__ uint32_t pre[kTileMaxWords];
+                                                     int64_t n, int nwords, const uint32_t* blockBits,
+                                                     const int64_t* segBase, uint32_t* segTile, uint32_t* segCnt,
+                                                     uint32_t* segStart, uint32_t* segInst, uint32_t* segTotal,
+                                                     uint32_t* fill, int64_t* blockE, int64_t* blockI) {
+  extern __shared__ uint32_t bits[];
+  uint32_t* pre = bits + nwords;
   __shared__ uint32_t cntL[kWaves][kTileLdsSegs];
   const int64_t b = blockIdx.x;
-  tileBitmap(rowPtr, cols, perm, pos, bIdx, bPos, n, b, nwords, bits, pre);
+  for (int k = threadIdx.x; k < nwords; k += kBlock) bits[k] = blockBits[b * nwords + k];
+  __syncthreads();
+  tilePrefix(nwords, bits, pre);
   const int wave = threadIdx.x >> 6, lane = __lane_id();
   const int64_t base = segBase[b];
   const bool inLds = segBase[b + 1] - base <= kTileLdsSegs;
@@ -2144,17 +2151,20 @@ template <typename VT>
 __global__ void __launch_bounds__(kBlock) kTileFill(const int64_t* rowPtr, const int32_t* cols, const VT* vals,
                                                     const uint32_t* perm, const uint32_t* pos, const uint32_t* bIdx,
                                                     const uint32_t* bPos, int64_t n, int nwords,
+                                                    const uint32_t* blockBits,
                                                     const int64_t* segBase, const uint32_t* segTile,
                                                     const uint32_t* segStart, const uint32_t* segInst,
                                                     const uint32_t* segTotal, uint32_t* fill,
                                                     const int64_t* blockE, const int64_t* blockI, uint32_t* tIdx,
                                                     VT* tVal, uint2* inst, int stageMin, const float* lo,
                                                     float* tLo) {
-  __shared__ uint32_t bits[kTileMaxWords];
-  __shared__ uint32_t pre[kTileMaxWords];
+  extern __shared__ uint32_t bits[];
+  uint32_t* pre = bits + nwords;
   __shared__ uint32_t fillL[kWaves][kTileLdsSegs];
   const int64_t b = blockIdx.x;
-  tileBitmap(rowPtr, cols, perm, pos, bIdx, bPos, n, b, nwords, bits, pre);
+  for (int k = threadIdx.x; k < nwords; k += kBlock) bits[k] = blockBits[b * nwords + k];
+  __syncthreads();
+  tilePrefix(nwords, bits, pre);
   const int wave = threadIdx.x >> 6, lane = __lane_id();
   const int64_t base = segBase[b], eb = blockE[b];
   const bool inLds = segBase[b + 1] - base <= kTileLdsSegs;
@@ -4428,7 +4438,8 @@ void launchSigmaPermF32(const int64_t* rp, const int32_t* cols, const float* val
 
 void TiledHam::release() {
   for (DevMem* m : {&segBase, &segTile, &segCnt, &segStart, &segInst, &segTotal, &fill, &blockE, &blockI, &idx, &vals,
-                    &lo, &inst, &order, &blockOf, &bigI, &smallI, &lead, &groups, &symInst, &unitStart, &units})
+                    &lo, &inst, &tileBits, &order, &blockOf, &bigI, &smallI, &lead, &groups, &symInst, &unitStart,
+                    &units})
     m->release();
   n = -1;
   hasLo = false;
@@ -4444,7 +4455,7 @@ size_t tiledHamBytes(int64_t n, int64_t nnz, bool f32) {
   // bytes) with at most one segment per 64 entries or per block
   const int64_t segs = nnz / 64 + blocks;
   return (size_t)nnz * (4 + (f32 ? 4 : 8)) + (size_t)(nnz / 32 + segs) * 16 + (size_t)segs * 88 +
-         (size_t)(blocks + 1) * 40;
+         (size_t)(blocks + 1) * (40 + (size_t)((2 * n + kTileCols - 1) / kTileCols + 31) / 32 * 4);
 }
 
 bool buildTiledHam(TiledHam& T, const int64_t* rowPtr, const int32_t* cols, const double* vals64,
@@ -4465,7 +4476,10 @@ bool buildTiledHam(TiledHam& T, const int64_t* rowPtr, const int32_t* cols, cons
   T.segBase.reserve((size_t)(blocks + 1) * 8);
   int64_t* segBase = T.segBase.as<int64_t>();
   HIP_CHECK(hipMemsetAsync(segBase + blocks, 0, 8, s));
-  kTileMark<<<grid, kBlock, 0, s>>>(rowPtr, cols, perm, pos, bIdx, bPos, n, nwords, segBase);
+  T.tileBits.reserve((size_t)blocks * nwords * 4);
+  uint32_t* tileBits = T.tileBits.as<uint32_t>();
+  const size_t ldsBits = (size_t)nwords * 4;
+  kTileMark<<<grid, kBlock, ldsBits, s>>>(rowPtr, cols, perm, pos, bIdx, bPos, n, nwords, segBase, tileBits);
   HIP_CHECK(hipGetLastError());
   exclusiveScanI64(segBase, blocks + 1, ws, s);
   int64_t S = 0;
@@ -4485,10 +4499,10 @@ bool buildTiledHam(TiledHam& T, const int64_t* rowPtr, const int32_t* cols, cons
   int64_t* blockI = T.blockI.as<int64_t>();
   HIP_CHECK(hipMemsetAsync(blockE + blocks, 0, 8, s));
   HIP_CHECK(hipMemsetAsync(blockI + blocks, 0, 8, s));
-  kTileCount<<<grid, kBlock, 0, s>>>(rowPtr, cols, perm, pos, bIdx, bPos, n, nwords, segBase,
-                                     T.segTile.as<uint32_t>(), T.segCnt.as<uint32_t>(), T.segStart.as<uint32_t>(),
-                                     T.segInst.as<uint32_t>(), T.segTotal.as<uint32_t>(), T.fill.as<uint32_t>(),
-                                     blockE, blockI);
+  kTileCount<<<grid, kBlock, 2 * ldsBits, s>>>(
+      rowPtr, cols, perm, pos, bIdx, bPos, n, nwords, tileBits, segBase, T.segTile.as<uint32_t>(),
+      T.segCnt.as<uint32_t>(), T.segStart.as<uint32_t>(), T.segInst.as<uint32_t>(), T.segTotal.as<uint32_t>(),
+      T.fill.as<uint32_t>(), blockE, blockI);
   HIP_CHECK(hipGetLastError());
   exclusiveScanI64(blockE, blocks + 1, ws, s);
   exclusiveScanI64(blockI, blocks + 1, ws, s);
@@ -4507,20 +4521,16 @@ bool buildTiledHam(TiledHam& T, const int64_t* rowPtr, const int32_t* cols, cons
   T.inst.reserve((size_t)(I + kTileInstPad) * 8);
   HIP_CHECK(hipMemsetAsync(T.inst.as<uint2>() + I, 0, (size_t)kTileInstPad * 8, s));
   if (f32)
-    kTileFill<float><<<grid, kBlock, 0, s>>>(rowPtr, cols, vals32, perm, pos, bIdx, bPos, n, nwords, segBase,
-                                             T.segTile.as<uint32_t>(), T.segStart.as<uint32_t>(),
-                                             T.segInst.as<uint32_t>(),
-                                             T.segTotal.as<uint32_t>(), T.fill.as<uint32_t>(), blockE, blockI,
-                                             T.idx.as<uint32_t>(), T.vals.as<float>(), T.inst.as<uint2>(),
-                                             stageMin, withLo ? valsLo : nullptr,
-                                             withLo ? T.lo.as<float>() : nullptr);
+    kTileFill<float><<<grid, kBlock, 2 * ldsBits, s>>>(
+        rowPtr, cols, vals32, perm, pos, bIdx, bPos, n, nwords, tileBits, segBase, T.segTile.as<uint32_t>(),
+        T.segStart.as<uint32_t>(), T.segInst.as<uint32_t>(), T.segTotal.as<uint32_t>(), T.fill.as<uint32_t>(), blockE,
+        blockI, T.idx.as<uint32_t>(), T.vals.as<float>(), T.inst.as<uint2>(), stageMin, withLo ? valsLo : nullptr,
+        withLo ? T.lo.as<float>() : nullptr);
   else
-    kTileFill<double><<<grid, kBlock, 0, s>>>(rowPtr, cols, vals64, perm, pos, bIdx, bPos, n, nwords, segBase,
-                                              T.segTile.as<uint32_t>(), T.segStart.as<uint32_t>(),
-                                              T.segInst.as<uint32_t>(),
-                                              T.segTotal.as<uint32_t>(), T.fill.as<uint32_t>(), blockE, blockI,
-                                              T.idx.as<uint32_t>(), T.vals.as<double>(), T.inst.as<uint2>(),
-                                              stageMin, nullptr, nullptr);
+    kTileFill<double><<<grid, kBlock, 2 * ldsBits, s>>>(
+        rowPtr, cols, vals64, perm, pos, bIdx, bPos, n, nwords, tileBits, segBase, T.segTile.as<uint32_t>(),
+        T.segStart.as<uint32_t>(), T.segInst.as<uint32_t>(), T.segTotal.as<uint32_t>(), T.fill.as<uint32_t>(), blockE,
+        blockI, T.idx.as<uint32_t>(), T.vals.as<double>(), T.inst.as<uint2>(), stageMin, nullptr, nullptr);
   HIP_CHECK(hipGetLastError());
   kTileRunBits<<<grid, kBlock, 0, s>>>(T.inst.as<uint2>(), blockI, blockE, T.idx.as<uint32_t>());
   HIP_CHECK(hipGetLastError());
