@@ -282,7 +282,7 @@ double Engine::ptDeterministic(const double* dCi, double e0, double eps2, double
     ensureTable(n);
     ptTables();
     const DevSystem P = ptSystem();
-    const int slices = ptSlices(n, hs.nelec);
+    const int slices = pairSlices(n, hs.nelec);
     const int64_t nc = n * slices;
     ptCounts.reserve((size_t)(nc + 1) * 8);
     int64_t* cnt = ptCounts.as<int64_t>();
@@ -385,7 +385,7 @@ double Engine::ptSemistochastic(const double* dCi, double e0, double eps2, doubl
   ensureTable(n);
   ptTables();
   const DevSystem P = ptSystem();
-  const int slices = ptSlices(Nmc, hs.nelec);
+  const int slices = pairSlices(Nmc, hs.nelec);
   ptCounts.reserve(((size_t)Nmc * slices + 1) * 8);
   ptOut.reserve(64);
   int64_t* cnt = ptCounts.as<int64_t>();

@@ -28,13 +28,13 @@ void launchCmax(const double* ci, int nroots, int64_t ld, int64_t n, double* cma
 // Screens the source determinants [begin, end) of `dets` (the whole
 // variational space is probed for membership).
 // Deterministic EN-PT2 candidates of sources [0, n) (SHCI/SHCIgetdeterminants.cpp:40-171):
-// each cut into `slices` parts (ptSlices): with fillStart == nullptr the count
+// each cut into `slices` parts (pairSlices): with fillStart == nullptr the count
 // pass writes counts[src * slices + part]; otherwise the fill pass writes each
 // part's candidates (determinants outD, numerators H_ai c_i outN) from
 // fillStart on, a source's by electron pairs as the reference generates them.
 // Only candidates outside the membership table and in partition `part` of
 // `nparts` are kept.  dense: buildDenseHeatBath's two tables.
-int ptSlices(int64_t nsrc, int nelec);
+int pairSlices(int64_t nsrc, int nelec);
 void buildDenseHeatBath(const DevSystem& S, DevMem* dense, hipStream_t s);
 void launchPtGen(const DevSystem& S, const uint64_t* dets, int64_t n, const double* ci, double eps2,
                  const int32_t* table, uint64_t slots, uint32_t nparts, uint32_t part, int slices, const DevMem* dense,

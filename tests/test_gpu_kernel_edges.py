@@ -71,6 +71,22 @@ def test_pt_candidates_of_few_sources(case, n, eps2, tmp_path):
     np.testing.assert_allclose(got[:2], ref[:2], rtol=1e-11, atol=0)
 
 
+@pytest.mark.parametrize("eps", [1e-5, 3e-3, 10.0])
+@pytest.mark.parametrize("case,n", [("w1", 1), ("w1", 3), ("w1", 1200), ("w2", 1), ("w2", 65)])
+def test_screening_of_few_sources(case, n, eps, tmp_path):
+    """Sources cut into parts and whole, candidates by the queue's 64s and its
+    rest, none at all: the same new determinants as the oracle's, each once."""
+    from dice_amd import shci
+    path, occ, W = _system(case, tmp_path)
+    dets = _space(path, occ, n, W)
+    ci = np.linspace(1.0, 0.1, n)
+    s = shci.System.from_fcidump(path)
+    s.set_dets(dets)
+    got = s.get_determinants_variational(ci, eps)
+    want = OracleSystem(path).screen(dets, ci, eps)
+    np.testing.assert_array_equal(got, want)
+
+
 @pytest.mark.parametrize("n", [3, 8, 257, 1500])
 @pytest.mark.parametrize("roots", [1, 2, 9])
 def test_davidson_subspaces(n, roots, tmp_path):
