@@ -3645,116 +3645,144 @@ __global__ void __launch_bounds__(kBlock) kScaleSum(double* dst, const double* _
 // to even) are rotated at once, m'-1 steps per sweep, so a sweep needs
 // m'-1 rounds of barriers instead of m(m-1)/2.  Another rotation order than
 // jacobiWave's, so the eigenpairs agree with it to rounding, not bit for bit;
-// used by the block Davidson.
-__global__ void __launch_bounds__(64) kJacobiRR(const double* A, int m, double* w, double* V) {
+// used by the block Davidson.  A chain of steps again: a step's rotations (two
+// divisions and two roots), then all elements.  Thread (R, C) has the four
+// elements of the row pair R and the column pair C, which no other pair mixes,
+// and applies C's rotation and then R's to them in registers (16 x 16 threads
+// cover the largest m), so a step is two barriers and one LDS round trip, not
+// four passes of one wave over the matrix.  m = 8..24: 209 -> 102 us.
+__global__ void __launch_bounds__(kBlock) kJacobiRR(const double* A, int m, double* w, double* V) {
+  static_assert(kJacobiMax <= 32 && kBlock == 256, "a thread per pair of pairs");
   __shared__ double a[kJacobiMax * kJacobiMax], v[kJacobiMax * kJacobiMax];
-  __shared__ double rc[kJacobiMax / 2], rs[kJacobiMax / 2];
-  __shared__ int rp[kJacobiMax / 2], rq[kJacobiMax / 2];
-  __shared__ double sOff;
+  __shared__ double rc[16], rs[16];
+  __shared__ int rp[16], rq[16];
+  __shared__ int rk[16];  // 1: rotate, 0: leave, -1: zero the pivot only
   __shared__ int order[kJacobiMax];
-  const int lane = threadIdx.x;
+  const int tid = threadIdx.x;
   const int mm = (m + 1) & ~1, half = mm / 2;
-  for (int q = lane; q < m * m; q += 64) {
+  for (int q = tid; q < m * m; q += kBlock) {
     a[q] = A[q];
-    v[q] = 0.0;
+    v[q] = q / m == q % m ? 1.0 : 0.0;
   }
-  __syncthreads();
-  if (lane < m) v[lane * m + lane] = 1.0;
+  const int R = tid >> 4, C = tid & 15;
+  const bool mine = R < half && C < half;
+  const int k0 = 2 * R, k1 = 2 * R + 1;  // this thread's rows of v (pair C)
   __syncthreads();
   for (int sweep = 0; sweep < 100; sweep++) {
-    double part = 0.0;
-    for (int t = lane; t < m * m; t += 64) {
-      const int p = t / m, q = t % m;
-      if (q > p) part += fabs(a[t]);
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
-    if (lane == 0) sOff = part;
-    __syncthreads();
-    if (sOff == 0.0) break;
+    int off = 0;
+    for (int t = tid; t < m * m; t += kBlock)
+      if (t % m > t / m && a[t] != 0.0) off = 1;
+    if (!__syncthreads_or(off)) break;
     for (int step = 0; step < mm - 1; step++) {
-      if (lane < half) {
+      if (tid < half) {
         // round-robin: player 0 fixed, the others rotate by step
-        const int i = lane, j = mm - 1 - lane;
-        int p = i == 0 ? 0 : (i - 1 + step) % (mm - 1) + 1;
-        int q = (j - 1 + step) % (mm - 1) + 1;
+        int p = 0, q = mm - 2 - tid + step;
+        if (tid > 0) {
+          p = tid - 1 + step;
+          p = (p >= mm - 1 ? p - (mm - 1) : p) + 1;
+        }
+        q = (q >= mm - 1 ? q - (mm - 1) : q) + 1;
         if (p > q) {
           const int t = p;
           p = q;
           q = t;
         }
         double c = 1.0, sn = 0.0;
-        int pp = -1;
+        int kind = 0;
         if (q < m) {
           const double apq = a[p * m + q], app = a[p * m + p], aqq = a[q * m + q];
           const double g = 100.0 * fabs(apq);
           if (sweep > 3 && fabs(app) + g == fabs(app) && fabs(aqq) + g == fabs(aqq)) {
-            pp = -2;  // negligible: zero it without a rotation
+            kind = -1;  // negligible: zero it without a rotation
           } else if (apq != 0.0) {
             const double theta = (aqq - app) / (2.0 * apq);
             const double t = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
             c = 1.0 / sqrt(t * t + 1.0);
             sn = t * c;
-            pp = p;
+            kind = 1;
           }
         }
-        rp[lane] = pp == -2 ? -2 - p : pp;
-        rq[lane] = q;
-        rc[lane] = c;
-        rs[lane] = sn;
+        rp[tid] = p;
+        rq[tid] = q;
+        rk[tid] = kind;
+        rc[tid] = c;
+        rs[tid] = sn;
       }
       __syncthreads();
-      // columns p, q of every row k (a), then rows p, q and columns of v
-      for (int t = lane; t < half * m; t += 64) {
-        const int r = t / m, k = t % m;
-        const int p = rp[r], q = rq[r];
-        if (p < 0) continue;
-        const double c = rc[r], sn = rs[r];
-        const double akp = a[k * m + p], akq = a[k * m + q];
-        a[k * m + p] = c * akp - sn * akq;
-        a[k * m + q] = sn * akp + c * akq;
-      }
-      __syncthreads();
-      for (int t = lane; t < half * m; t += 64) {
-        const int r = t / m, k = t % m;
-        const int p = rp[r], q = rq[r];
-        if (p < 0) continue;
-        const double c = rc[r], sn = rs[r];
-        const double apk = a[p * m + k], aqk = a[q * m + k];
-        a[p * m + k] = c * apk - sn * aqk;
-        a[q * m + k] = sn * apk + c * aqk;
-        const double vkp = v[k * m + p], vkq = v[k * m + q];
-        v[k * m + p] = c * vkp - sn * vkq;
-        v[k * m + q] = sn * vkp + c * vkq;
-      }
-      __syncthreads();
-      if (lane < half) {
-        int p = rp[lane];
-        const int q = rq[lane];
-        if (p <= -2) p = -2 - p;  // negligible pair
-        if (p >= 0 && q < m) {
-          a[p * m + q] = 0.0;
-          a[q * m + p] = 0.0;
+      if (mine) {
+        const int p = rp[R], q = rq[R], kindR = rk[R];
+        const int pc = rp[C], qc = rq[C], kindC = rk[C];
+        if (kindR != 0 || kindC != 0) {
+          // q or qc == m: the pair of the one left over (odd m), no such row
+          const bool hasQ = q < m, hasQc = qc < m;
+          double pp = a[p * m + pc], pq = 0.0, qp = 0.0, qq = 0.0;
+          if (hasQc) pq = a[p * m + qc];
+          if (hasQ) qp = a[q * m + pc];
+          if (hasQ && hasQc) qq = a[q * m + qc];
+          if (kindC > 0) {
+            const double c = rc[C], sn = rs[C];
+            const double x = c * pp - sn * pq, y = sn * pp + c * pq;
+            pp = x;
+            pq = y;
+            const double z = c * qp - sn * qq, u = sn * qp + c * qq;
+            qp = z;
+            qq = u;
+            if (k0 < m) {
+              const double vp = v[k0 * m + pc], vq = v[k0 * m + qc];
+              v[k0 * m + pc] = c * vp - sn * vq;
+              v[k0 * m + qc] = sn * vp + c * vq;
+            }
+            if (k1 < m) {
+              const double vp = v[k1 * m + pc], vq = v[k1 * m + qc];
+              v[k1 * m + pc] = c * vp - sn * vq;
+              v[k1 * m + qc] = sn * vp + c * vq;
+            }
+          }
+          if (kindR > 0) {
+            const double c = rc[R], sn = rs[R];
+            const double x = c * pp - sn * qp, y = sn * pp + c * qp;
+            pp = x;
+            qp = y;
+            const double z = c * pq - sn * qq, u = sn * pq + c * qq;
+            pq = z;
+            qq = u;
+          }
+          if (R == C) pq = qp = 0.0;
+          a[p * m + pc] = pp;
+          if (hasQc) a[p * m + qc] = pq;
+          if (hasQ) a[q * m + pc] = qp;
+          if (hasQ && hasQc) a[q * m + qc] = qq;
         }
       }
       __syncthreads();
     }
   }
-  if (lane == 0) {
-    for (int i = 0; i < m; i++) order[i] = i;
-    for (int i = 1; i < m; i++) {  // stable insertion sort by eigenvalue
-      const int o = order[i];
-      int j = i;
-      while (j > 0 && a[order[j - 1] * m + order[j - 1]] > a[o * m + o]) {
-        order[j] = order[j - 1];
-        j--;
+  // stable order by eigenvalue: by rank, or (NaNs have none) by insertion
+  if (__syncthreads_or(tid < m && isnan(a[tid * m + tid]))) {
+    if (tid == 0) {
+      for (int i = 0; i < m; i++) order[i] = i;
+      for (int i = 1; i < m; i++) {
+        const int o = order[i];
+        int j = i;
+        while (j > 0 && a[order[j - 1] * m + order[j - 1]] > a[o * m + o]) {
+          order[j] = order[j - 1];
+          j--;
+        }
+        order[j] = o;
       }
-      order[j] = o;
     }
+  } else if (tid < m) {
+    const double d = a[tid * m + tid];
+    int rank = 0;
+    for (int j = 0; j < m; j++) {
+      const double e = a[j * m + j];
+      rank += e < d || (e == d && j < tid);
+    }
+    order[rank] = tid;
   }
   __syncthreads();
-  if (lane < m) w[lane] = a[order[lane] * m + order[lane]];
-  for (int q = lane; q < m * m; q += 64) {
+  if (tid < m) w[tid] = a[order[tid] * m + order[tid]];
+  for (int q = tid; q < m * m; q += kBlock) {
     const int k = q / m, j = q % m;
     V[k * m + j] = v[k * m + order[j]];
   }
@@ -4863,7 +4891,7 @@ void launchSymmetrizeUpper(const double* G, int m, double* A, hipStream_t s) {
 
 void launchJacobiRR(const double* A, int m, double* w, double* V, hipStream_t s) {
   if (m > kJacobiMax) throw HipError("launchJacobiRR: subspace too large");
-  kJacobiRR<<<1, 64, 0, s>>>(A, m, w, V);
+  kJacobiRR<<<1, kBlock, 0, s>>>(A, m, w, V);
   HIP_CHECK(hipGetLastError());
 }
 
