@@ -1109,7 +1109,7 @@ std::vector<double> Engine::davidsonBlock(double* dX0, int nr, double tol, int& 
   reserveKeep(bdX, (size_t)N * nr * 8);
   reserveKeep(bdHX, (size_t)N * nr * 8);
   reserveKeep(bdR, (size_t)N * nr * 8);
-  reserveKeep(bdSmall, (size_t)8 * 4096 * 8);
+  reserveKeep(bdSmall, (size_t)7 * 4096 * 8);
   reserveKeep(dvPart, (size_t)16 * 256 * 64 * 8);  // largest Gram: 16 tiles x 256 blocks x 8 x 8
   reserveKeep(dvScal, 64 * 8);
   // x in alpha- and beta-major order, up to 8 interleaved vectors
@@ -1117,13 +1117,12 @@ std::vector<double> Engine::davidsonBlock(double* dX0, int nr, double tol, int& 
   reserveKeep(sigmaCounter, 256);
   if (!bdHost) HIP_CHECK(hipHostMalloc((void**)&bdHost, 64 * 8, hipHostMallocDefault));
   double* sm = bdSmall.as<double>();
-  double* G = sm;                 // m x m Gram matrix (upper triangle used)
-  double* A = sm + 4096;          // symmetrised
-  double* C = sm + 2 * 4096;      // eigenvectors (row-major, column j = vector j)
-  double* w = sm + 3 * 4096;      // eigenvalues
-  double* Cn = sm + 4 * 4096;     // first nr (or keep) columns of C
-  double* coef = sm + 5 * 4096;   // V^T T
-  double* nrm = sm + 6 * 4096;    // residual norms^2 (nr), then correction norms^2
+  double* A = sm;                 // m x m Gram matrix V^T S, upper triangle mirrored
+  double* C = sm + 4096;          // eigenvectors (row-major, column j = vector j)
+  double* w = sm + 2 * 4096;      // eigenvalues
+  double* Cn = sm + 3 * 4096;     // first nr (or keep) columns of C
+  double* coef = sm + 4 * 4096;   // V^T T
+  double* nrm = sm + 5 * 4096;    // residual norms^2 (nr), then correction norms^2
   double* sc = dvScal.as<double>();
   int cur = 0;
   double* V = bdV[0].as<double>();
@@ -1141,7 +1140,7 @@ std::vector<double> Engine::davidsonBlock(double* dX0, int nr, double tol, int& 
     for (int j = 0; j < b; j++) launchNorm2(col(Tm, j), N, nrm + 16 + j, dvPart, s);
     if (m > 0)
       for (int pass = 0; pass < 2; pass++) {
-        launchGramTiled(V, m, Tm, b, N, N, coef, dvPart, s);
+        launchGramTiled(V, m, Tm, b, N, N, false, coef, dvPart, s);
         launchGemmTS(V, m, coef, b, N, N, Tm, N, -1.0, 1.0, s);
       }
     for (int j = 0; j < b; j++) {
@@ -1168,8 +1167,7 @@ std::vector<double> Engine::davidsonBlock(double* dX0, int nr, double tol, int& 
   auto body = [&](int m0, int b) {
     const int m = m0 + b;
     sigma(col(V, m0), col(S, m0), b, N, exactSigma);
-    launchGramTiled(V, m, S, m, N, N, G, dvPart, s);
-    launchSymmetrizeUpper(G, m, A, s);
+    launchGramTiled(V, m, S, m, N, N, true, A, dvPart, s);
     launchJacobiRR(A, m, w, C, s);
     launchSubMatrix(C, m, m, nr, Cn, s);
     launchGemmTS(V, m, Cn, nr, N, N, X, N, 1.0, 0.0, s);

@@ -334,8 +334,9 @@ void launchGram(const double* A, int ma, const double* B, int mb, int64_t n, int
                 DevMem& partial, hipStream_t s);
 // out[i*cols + j] = C[i*ldc + j] for i < rows, j < cols (small matrices)
 void launchSubMatrix(const double* C, int ldc, int rows, int cols, double* out, hipStream_t s);
-// G[i*mb + j] = A[:,i] . B[:,j] for ma, mb <= 64 (8 x 8 tiles; fixed-order sums)
-void launchGramTiled(const double* A, int ma, const double* B, int mb, int64_t n, int64_t ld, double* G,
+// G[i*mb + j] = A[:,i] . B[:,j] for ma, mb <= 64 (8 x 8 tiles; fixed-order sums);
+// upper (ma == mb): of i <= j only, mirrored
+void launchGramTiled(const double* A, int ma, const double* B, int mb, int64_t n, int64_t ld, bool upper, double* G,
                      DevMem& partial, hipStream_t s);
 // out[:, j] = alpha * sum_l A[:, l] W[l*mb + j] + beta * out[:, j] for j < mb
 // (W row-major ma x mb on device, ma, mb <= 64); out must not overlap A
@@ -356,8 +357,6 @@ void launchNorm2(const double* x, int64_t n, double* out, DevMem& partial, hipSt
 void launchScaleInto(double* dst, const double* src, const double* nrm2, int64_t n, hipStream_t s);
 // x += alpha * y
 void launchAxpy(double* x, const double* y, double alpha, int64_t n, hipStream_t s);
-// A[i*m+j] = G[min(i,j)*m + max(i,j)]  (upper triangle mirrored)
-void launchSymmetrizeUpper(const double* G, int m, double* A, hipStream_t s);
 // symmetric eigen-decomposition of the m x m matrix (row-major) by Jacobi
 // sweeps with the rotations in round-robin order (disjoint pairs at once),
 // eigenvalues ascending in w, eigenvectors in the columns of V (block Davidson)
