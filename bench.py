@@ -14,7 +14,7 @@ variational iteration over the timed steps.
 The roofline object is the sigma = H x kernel of the Davidson, timed with
 HIP events on the library's stream over the timed steps.  The Hamiltonian's
 lower triangle alone is stored (the library's default for the single-vector
-Davidson): kSigmaTiledSym over a tiled copy of it (256-row blocks of the
+Davidson): kSigmaTiledSym over a tiled copy of it (super blocks of 1024
 alpha-major relabelled rows, entries grouped by 1024-column tiles), each
 stored element applied to its row and, in 64-bit fixed point, to its
 column, with its x permutation and the final addition into y.  Achieved
@@ -624,7 +624,7 @@ def main():
         },
         "roofline": {
             "bound": "hbm",
-            "kernel": "kSigmaTiledSym (sigma = H x over the stored lower triangle: 256-row blocks of the "
+            "kernel": "kSigmaTiledSym (sigma = H x over the stored lower triangle: super blocks of 1024 "
                       "alpha-major relabelled rows, entries grouped by 1024-column tiles, each entry applied to its "
                       "row and, in 64-bit fixed point, to its column)",
             "achieved": round(achieved, 1),
