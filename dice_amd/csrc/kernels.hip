@@ -680,7 +680,8 @@ __global__ void __launch_bounds__(kBlock) kPtGen(DevSystem S, const uint64_t* de
               }
               const int A = sSpin[wave][cI & 1][x], B = sSpin[wave][cJ & 1][y];
               hv = (same ? dense1 : dense0)[sStart[wave][q] + A * norb + B];
-              ok = (double)fabsf(hv) >= eps;
+              // (as the walk: an eps that is NaN, 0 / 0, cuts nothing off)
+              ok = !isnan(hv) && !((double)fabsf(hv) < eps);
               a = 2 * A + (cI & 1);
               b = 2 * B + (cJ & 1);
             } else {

@@ -71,6 +71,24 @@ def test_pt_candidates_of_few_sources(case, n, eps2, tmp_path):
     np.testing.assert_allclose(got[:2], ref[:2], rtol=1e-11, atol=0)
 
 
+@pytest.mark.parametrize("case,n", [("w1", 65), ("w2", 130)])
+def test_pt_candidates_of_zero_coefficients(case, n, tmp_path):
+    """eps2 0 and coefficients that are 0: their threshold |0 / 0| cuts no
+    double excitation off, so its external determinants are counted (with
+    numerators 0), from the lists and from the open orbitals alike."""
+    from dice_amd import shci
+    path, occ, W = _system(case, tmp_path)
+    dets = _space(path, occ, n, W)
+    s = shci.System.from_fcidump(path)
+    s.set_dets(dets)
+    c = np.random.default_rng(n).normal(size=n)
+    c[1:] = 0.0
+    e0 = s.energy(dets).min() - 2.0
+    got, ref = s.pt_deterministic(c, e0, 0.0), OracleSystem(path).pt_deterministic(dets, c, e0, 0.0)
+    assert got[2] == ref[2]
+    np.testing.assert_allclose(got[:2], ref[:2], rtol=1e-11, atol=0)
+
+
 @pytest.mark.parametrize("eps", [1e-5, 3e-3, 10.0])
 @pytest.mark.parametrize("case,n", [("w1", 1), ("w1", 3), ("w1", 1200), ("w2", 1), ("w2", 65)])
 def test_screening_of_few_sources(case, n, eps, tmp_path):
