@@ -632,6 +632,9 @@ void Engine::buildHamiltonian() {
   if (nDiag < n) launchEnergy(S, dets.as<uint64_t>() + nDiag * hs.W, n - nDiag, diag.as<double>() + nDiag, stream);
   nDiag = n;
   if (hamRows == n) return;
+  // captured block-Davidson iterations hold the addresses, sizes and launch
+  // shapes of the Hamiltonian that is replaced here (and of its copies)
+  clearGraphs();
   if (trev) {  // the adapted basis (also in direct mode: the E Hamiltonian is stored)
     buildTrev();
     hamRows = n;
@@ -1082,7 +1085,8 @@ void Engine::clearGraphs() {
 // 2 nr + 2 lowest Ritz vectors.  The iteration body after the host's choice
 // of corrections (SpMM, Gram matrix, eigensolve, Ritz vectors, residuals,
 // copy of Ritz values and residual norms to pinned host memory) is captured
-// once per (subspace size, block size) as a hipGraph and replayed.
+// once per (subspace size, block size) as a hipGraph and replayed, by later
+// calls too, until the Hamiltonian is built anew or a buffer here grows.
 std::vector<double> Engine::davidsonBlock(double* dX0, int nr, double tol, int& numIter, bool exactSigma) {
   const int64_t N = n;
   // subspace size: min(32, max(6 nr, nr + 16)) unless SHCI_BLOCK_MAXM (nr + 2 .. 32) sets it

@@ -507,6 +507,34 @@ def test_block_davidson_graph_replays_match_eager(systems):
         np.testing.assert_array_equal(x0, x1)
 
 
+@pytest.mark.parametrize("storage", ["half", "full"])
+def test_block_davidson_graphs_follow_the_hamiltonian(storage, systems, monkeypatch):
+    """One handle, Hamiltonians of one size after each other (another space,
+    denser and sparser, other values' precision, the first again): what graphs
+    replay is the Hamiltonian of the call, bit for bit as launched eagerly."""
+    monkeypatch.setenv("SHCI_STORAGE", storage)
+    path = systems["hub"][0]
+    held = _space("hub", systems, 4000, 1)
+    spaces = [held[:1500], held[2500:4000], held[500:2000]]
+    n = 1500
+    res = {}
+    for graphs in (False, True):
+        g = _gpu(path)
+        out = []
+        for which, prec in ((0, 0), (1, 0), (2, 0), (0, 0), (0, 1), (0, 0)):
+            g.set_options(precision=prec, davidson_block=True, hip_graphs=graphs)
+            g.set_dets(spaces[which])
+            g.make_hamiltonian()
+            x0 = np.random.default_rng(which).normal(size=(n, 2))
+            x0[0] += 5.0
+            out.append(g.davidson(x0, tol=1e-4))
+        res[graphs] = out
+    for (e0, x0, i0), (e1, x1, i1) in zip(res[False], res[True]):
+        assert i0 == i1
+        np.testing.assert_array_equal(e0, e1)
+        np.testing.assert_array_equal(x0, x1)
+
+
 def test_autotuned_sigma_matches_default(systems, monkeypatch):
     """With autotune on (both triangles stored: the row copy's launch shapes),
     the Hamiltonian build times every launch shape and keeps the fastest;
