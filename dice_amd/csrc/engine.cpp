@@ -269,7 +269,9 @@ DevSystem Engine::ptSystem() const {
 }
 
 void Engine::ptTables() {
-  if (!ptDense[0].p) buildDenseHeatBath(S, ptDense, stream);
+  if (ptDenseReady) return;
+  buildDenseHeatBath(S, ptDense, stream);
+  ptDenseReady = true;  // (not set when an allocation or a launch failed)
 }
 
 double Engine::ptDeterministic(const double* dCi, double e0, double eps2, double* psi1Norm, int64_t* nExternal,

@@ -202,6 +202,7 @@ struct Engine {
   // candidates are processed in hash partitions sized to the free memory
   DevMem ptCounts, ptKeys, ptNum, ptIdx, ptOut, ptPartial, ptStartCnt, ptStarts;
   DevMem ptDense[2];  // dense copies of the heat-bath lists, made by the first PT call
+  bool ptDenseReady = false;
   void ptTables();
   double ptDeterministic(const double* dCi, double e0, double eps2, double* psi1Norm, int64_t* nExternal,
                          int* nPartitions = nullptr);

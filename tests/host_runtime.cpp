@@ -116,7 +116,7 @@ void submit(Node n) {
 
 extern "C" {
 // what tests ask
-void fake_fail_in(int k) { failIn = k; }  // the k-th allocation from now fails
+void fake_fail_in(int k) { failIn = k; }  // allocations fail from the k-th on (0: none)
 void fake_set_free(uint64_t bytes) { freeBytes = bytes; }
 int fake_stale() { return stale; }  // replayed arguments whose allocation was freed
 int fake_captures() { return captures; }
@@ -169,7 +169,8 @@ int hipLaunchKernel(const void* host, Dim grid, Dim, void** args, size_t, void*)
   return 0;
 }
 int hipMalloc(void** p, size_t bytes) {
-  if (failIn > 0 && --failIn == 0) return kOutOfMemory;
+  if (failIn == 1) return kOutOfMemory;
+  if (failIn > 1) failIn--;
   static int ids = 0;
   *p = calloc(1, bytes ? bytes : 1);
   blocks[(uintptr_t)*p] = Block{bytes, ++ids, true};

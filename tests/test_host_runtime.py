@@ -76,3 +76,29 @@ after = solve()
 assert F.fake_stale() == 0
 assert after == before + first  # captured anew
 """ % change, tmp_path, SHCI_STORAGE=storage)
+
+
+def test_pt_after_a_failed_allocation(host_runtime, tmp_path):
+    """Whichever allocation of a PT call fails, the next call on the handle has
+    both dense heat-bath tables, filled."""
+    host_runtime("""
+space = dets(5, 1)
+c = np.full(5, 5 ** -0.5)
+failed = 0
+for k in range(1, 20):
+    s = shci.System.from_fcidump(path)
+    s.set_dets(space)
+    fills = F.fake_launches(b"kDenseHeatBath")
+    F.fake_fail_in(k)
+    try:
+        s.pt_deterministic(c, -1.0, 1e-3)
+    except shci.ShciError:
+        failed += 1
+    F.fake_fail_in(0)
+    calls = F.fake_launches(b"kPtGen")
+    s.pt_deterministic(c, -1.0, 1e-3)
+    assert F.fake_launches(b"kPtGen") > calls
+    assert F.fake_last_arg(b"kPtGen", 15) and F.fake_last_arg(b"kPtGen", 16), k  # dense0, dense1
+    assert F.fake_launches(b"kDenseHeatBath") >= fills + 2, k
+assert failed >= 4  # (the tables, the counts, and what the call itself holds)
+""", tmp_path)
