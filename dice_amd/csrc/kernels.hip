@@ -2807,8 +2807,13 @@ __global__ void kGatherPermMax(const double* __restrict__ x, const uint32_t* __r
   double m = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nx; i += (int64_t)gridDim.x * blockDim.x) {
     const double v = x[i < n ? perm[i] : bPerm[i - n]];
-    xP[i] = fabs(v) <= DBL_MAX ? (XT)v : (XT)0;  // (with an infinite max|x| kSymFinish makes every sum NaN)
-    m = fmax(m, fabs(v));
+    // what has no place in a fixed point (NaN, infinite, beyond FP32 in its
+    // form) stays out of the sums; with an infinite max|x| kSymFinish makes
+    // every one of them NaN
+    const XT t = (XT)v;
+    const bool held = fabs((double)t) <= DBL_MAX;
+    xP[i] = held ? t : (XT)0;
+    m = fmax(m, held ? fabs(v) : (double)INFINITY);
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));

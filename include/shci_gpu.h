@@ -119,7 +119,9 @@ shci_status shci_get_hamiltonian_rows(shci_handle* h, int64_t row_begin, int64_t
 
 /* ---- sigma and Davidson --------------------------------------------------------------- */
 /* y[:, r] = H x[:, r] for r < k; x, y host, column-major n x k
- * (Hmult2::operator(), SHCI/Hmult.h:52-150). */
+ * (Hmult2::operator(), SHCI/Hmult.h:52-150).  With half storage an x[:, r] that
+ * holds a NaN, an infinity or (FP32 form) a value beyond FP32 makes all of
+ * y[:, r] NaN: its sums are in fixed point. */
 shci_status shci_sigma(shci_handle* h, const double* x, double* y, int k);
 /* Device-pointer variant on the handle's stream (stream = NULL) for callers
  * that keep vectors resident; returns after enqueueing.  ld >= n; d_y must

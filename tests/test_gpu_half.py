@@ -128,6 +128,36 @@ def test_half_storage_tiled_sigma_scales(tmp_path, monkeypatch):
     np.testing.assert_array_equal(h.hmult(np.zeros(len(dets))), np.zeros(len(dets)))
 
 
+@pytest.mark.parametrize("prec,bad", [(0, np.nan), (0, np.inf), (0, -np.inf), (1, np.nan), (1, np.inf), (1, 1e300)])
+def test_half_storage_tiled_sigma_of_non_finite_x(prec, bad, tmp_path, monkeypatch):
+    """No fixed point holds the products of an x that is NaN, infinite or (in
+    the FP32 form) beyond FP32's range: no row that it reaches comes back as a
+    finite number, and the next product is right again."""
+    from dice_amd import shci, synth
+    path = str(tmp_path / "FCIDUMP")
+    synth.write_molecular_fcidump(path, 0, 16, 8, 8, 64)
+    dets = _space(path, synth.hf_occupation(8, 8), 1500, 1)
+    monkeypatch.setenv("SHCI_STORAGE", "half")
+    h = shci.System.from_fcidump(path)
+    h.set_options(precision=prec)
+    h.set_dets(dets)
+    h.make_hamiltonian()
+    o = OracleSystem(path)
+    o.csr_append(dets)
+    x = np.random.default_rng(3).normal(size=len(dets))
+    y0 = h.hmult(x)
+    for at in (0, 700, len(dets) - 1):
+        unit = np.zeros(len(dets))
+        unit[at] = 1.0
+        reached = o.sigma(unit) != 0.0
+        reached[at] = False  # (its own row: the diagonal's product is in FP64)
+        assert reached.any()
+        xb = x.copy()
+        xb[at] = bad
+        assert not np.isfinite(h.hmult(xb)[reached]).any()
+    np.testing.assert_array_equal(h.hmult(x), y0)
+
+
 @pytest.mark.parametrize("mode", ["tiled", "rows"])
 @pytest.mark.parametrize("prec", [0, 1])
 def test_half_storage_run_matches_oracle(prec, mode, tmp_path, monkeypatch):
