@@ -876,7 +876,7 @@ void Engine::buildLowerTiled() {
   if (!relabel || !tiledOn || !lowerTiled || n == 0) return;
   const bool f32 = precision == 1;
   // (the FP32 form's copy holds the lo values too, for its exact sigma)
-  const size_t tiledCopy = tiledHamBytes(n, nnzOff, f32) + (f32 ? (size_t)nnzOff * 4 : 0);
+  const size_t tiledCopy = tiledHamBytes(n, nnzOff, f32, true) + (f32 ? (size_t)nnzOff * 4 : 0);
   const size_t base = (size_t)n * 4 + (size_t)n * 64;
   // permuted x (FP64 also in the FP32 form's exact sigma) and the
   // accumulators, plus bPos with split columns
@@ -929,7 +929,7 @@ void Engine::buildPermuted() {
   // and, with split columns, beta-major order too (plus bPos)
   const size_t xt = f32 ? 4 : 8, kmax = davidsonMode == 1 ? 8 : 1;
   const size_t rowsCopy = (size_t)nnzOff * (4 + (f32 ? 4 : 8)) + (size_t)(n + 1) * 8;
-  const size_t tiledCopy = tiledHamBytes(n, nnzOff, f32);
+  const size_t tiledCopy = tiledHamBytes(n, nnzOff, f32, false);
   const size_t base = (size_t)n * 4 + (size_t)n * 64;
   const size_t xPlain = (size_t)n * kmax * xt, xSplit = 2 * (size_t)n * kmax * xt + (size_t)n * 4;
   size_t freeB = 0, totalB = 0;

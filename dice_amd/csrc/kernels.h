@@ -274,9 +274,9 @@ struct TiledHam {
   int64_t unitCap = 0;
   void release();
 };
-// device bytes buildTiledHam needs for nnz entries over n rows (upper bound
-// on the per-segment tables)
-size_t tiledHamBytes(int64_t n, int64_t nnz, bool f32);
+// device bytes buildTiledHam needs for nnz entries over n rows, without or
+// with (sym) the half-storage order (upper bound on the per-segment tables)
+size_t tiledHamBytes(int64_t n, int64_t nnz, bool f32, bool sym);
 // Builds T from H in determinant order (rowPtr, cols, values: vals64 or, for
 // the FP32 form, vals32) through the alpha-major relabelling (perm: position
 // -> determinant, pos: determinant -> position) and, with bIdx / bPos given,

@@ -4597,14 +4597,16 @@ void TiledHam::release() {
 // the half-storage sigma's order of a tiled copy and its work units
 static void buildSymOrder(TiledHam& T, int bigMin, Workspace& ws, hipStream_t s);
 
-size_t tiledHamBytes(int64_t n, int64_t nnz, bool f32) {
+size_t tiledHamBytes(int64_t n, int64_t nnz, bool f32, bool sym) {
   const int64_t blocks = (n + kTileRows - 1) / kTileRows;
   // entries, one instruction per 32 entries at most on average plus one per
-  // segment (twice: the half-storage sigma's order), segment tables (88
-  // bytes) with at most one segment per 64 entries or per block
+  // segment, segment tables (48 bytes) with at most one segment per 64
+  // entries or per block, and the bitmaps of the blocks' tiles; sym: the
+  // instructions once more and 40 bytes per segment, in its own order
   const int64_t segs = nnz / 64 + blocks;
-  return (size_t)nnz * (4 + (f32 ? 4 : 8)) + (size_t)(nnz / 32 + segs) * 16 + (size_t)segs * 88 +
-         (size_t)(blocks + 1) * (40 + (size_t)((2 * n + kTileCols - 1) / kTileCols + 31) / 32 * 4);
+  const size_t bitmap = (size_t)((2 * n + kTileCols - 1) / kTileCols + 31) / 32 * 4;
+  return (size_t)nnz * (4 + (f32 ? 4 : 8)) + (size_t)(nnz / 32 + segs) * (sym ? 16 : 8) +
+         (size_t)segs * (sym ? 88 : 48) + (size_t)(blocks + 1) * ((sym ? 40 : 24) + bitmap);
 }
 
 bool buildTiledHam(TiledHam& T, const int64_t* rowPtr, const int32_t* cols, const double* vals64,

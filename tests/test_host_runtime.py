@@ -102,3 +102,20 @@ for k in range(1, 20):
     assert F.fake_launches(b"kDenseHeatBath") >= fills + 2, k
 assert failed >= 4  # (the tables, the counts, and what the call itself holds)
 """, tmp_path)
+
+
+def test_full_storage_needs_no_room_for_the_half_forms_order(host_runtime, tmp_path):
+    """Full storage takes the tiled copy when its own tables fit.  (No kernel
+    runs, so there are no entries: per determinant the inverse permutation,
+    x and 64 bytes of slack; per block of 256 rows a segment's tables and
+    instruction, offsets and a bitmap of up to 32 tiles.)"""
+    host_runtime("""
+n = 2000
+s = shci.System.from_fcidump(path)
+s.set_dets(dets(n, 1))
+blocks = (n + 255) // 256
+need = n * (4 + 8 + 64) + blocks * (8 + 48) + (blocks + 1) * (24 + 4)
+F.fake_set_free(need)
+s.make_hamiltonian()
+assert F.fake_launches(b"kTileFill") == 1
+""", tmp_path, SHCI_STORAGE="full")
