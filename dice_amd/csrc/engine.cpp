@@ -788,6 +788,7 @@ void Engine::buildHamiltonian() {
   buildPermuted();
   mark("relabel");
   HIP_CHECK(hipStreamSynchronize(stream));
+  tiled.releaseBuildTables(false);
   if (timing) {
     const double end = wallSeconds();
     std::string line = "  build n=" + std::to_string(n) + " (host ms / gpu ms):";
@@ -865,6 +866,7 @@ void Engine::buildLower(int64_t nOld) {
   permRows = -1;
   buildLowerTiled();
   HIP_CHECK(hipStreamSynchronize(stream));
+  tiled.releaseBuildTables(true);
 }
 
 // The tiled copy of the stored half, built from it through the alpha-major
@@ -934,8 +936,7 @@ void Engine::buildPermuted() {
   const size_t xPlain = (size_t)n * kmax * xt, xSplit = 2 * (size_t)n * kmax * xt + (size_t)n * 4;
   size_t freeB = 0, totalB = 0;
   freeB = deviceFreeBytes(&totalB);
-  const size_t have = freeB + permCols.bytes + permVals.bytes + permX.bytes + bPos.bytes + tiled.idx.bytes +
-                      tiled.vals.bytes + tiled.inst.bytes;
+  const size_t have = freeB + permCols.bytes + permVals.bytes + permX.bytes + bPos.bytes + tiled.heldBytes();
   // the tiled copy is built from the row-ordered one when both fit beside H;
   // when only the tiled copy fits it is built from H directly through the
   // permutation (a slower build)

@@ -272,7 +272,15 @@ struct TiledHam {
   // block), its instructions (symInst), tile groups and work units
   DevMem order, blockOf, bigI, smallI, lead, groups, symInst, unitStart, units;
   int64_t unitCap = 0;
+  std::vector<DevMem*> tables() {
+    return {&segBase, &segTile, &segCnt, &segStart, &segInst, &segTotal, &fill, &blockE, &blockI, &idx, &vals, &lo,
+            &inst, &tileBits, &order, &blockOf, &bigI, &smallI, &lead, &groups, &symInst, &unitStart, &units};
+  }
   void release();
+  // after a build (and what reads its tables): releases those that sigma does
+  // not read
+  void releaseBuildTables(bool sym);
+  size_t heldBytes();
 };
 // device bytes buildTiledHam needs for nnz entries over n rows, without or
 // with (sym) the half-storage order (upper bound on the per-segment tables)

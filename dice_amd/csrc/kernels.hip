@@ -4586,12 +4586,26 @@ void launchSigmaPermF32(const int64_t* rp, const int32_t* cols, const float* val
 }
 
 void TiledHam::release() {
-  for (DevMem* m : {&segBase, &segTile, &segCnt, &segStart, &segInst, &segTotal, &fill, &blockE, &blockI, &idx, &vals,
-                    &lo, &inst, &tileBits, &order, &blockOf, &bigI, &smallI, &lead, &groups, &symInst, &unitStart,
-                    &units})
-    m->release();
+  for (DevMem* m : tables()) m->release();
   n = -1;
   hasLo = false;
+}
+
+// With half storage only the next build would want them, and it begins by
+// releasing the copy; with full storage it fills the segment tables again, so
+// they stay, but not the bitmaps, whose size is quadratic in n.
+void TiledHam::releaseBuildTables(bool sym) {
+  tileBits.release();
+  if (!sym) return;
+  for (DevMem* m : {&segBase, &segTile, &segCnt, &segStart, &segInst, &segTotal, &fill, &blockI, &inst, &order, &blockOf,
+                    &bigI, &smallI, &lead, &unitStart})
+    m->release();
+}
+
+size_t TiledHam::heldBytes() {
+  size_t b = 0;
+  for (DevMem* m : tables()) b += m->bytes;
+  return b;
 }
 
 // the half-storage sigma's order of a tiled copy and its work units

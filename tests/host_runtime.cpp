@@ -41,7 +41,7 @@ std::vector<Node>* capture = nullptr;
 std::map<std::string, int> launched;
 std::map<std::string, std::vector<uint64_t>> lastArgs;
 int failIn = 0, captures = 0, stale = 0;
-size_t freeBytes = size_t(64) << 30;
+size_t freeBytes = size_t(256) << 30;
 Dim pushedGrid, pushedBlock;
 size_t pushedShared;
 void* pushedStream;

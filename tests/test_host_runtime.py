@@ -119,3 +119,30 @@ F.fake_set_free(need)
 s.make_hamiltonian()
 assert F.fake_launches(b"kTileFill") == 1
 """, tmp_path, SHCI_STORAGE="full")
+
+
+@pytest.mark.parametrize("storage,without,held", [
+    # what the product reads: entries (2), blockE, the ordered instructions,
+    # groups and units; beside them permPos, the sums and their scale
+    ("half", {"SHCI_HALF_SIGMA": "rows"}, 9),
+    # entries (2), instructions, blockE and blockI, and the segment tables (7),
+    # which the next build fills again
+    ("full", {"SHCI_SIGMA_LAYOUT": "rows"}, 12)])
+def test_tables_of_a_build_are_released(storage, without, held, host_runtime, tmp_path):
+    """Buffers that a built Hamiltonian with the tiled copy holds beyond one
+    without it."""
+    host_runtime("""
+def live():
+    s = shci.System.from_fcidump(path)
+    s.set_dets(dets(50, 1))
+    s.make_hamiltonian()
+    c = F.fake_live()
+    s.close()
+    return c
+tiled = live()
+os.environ.update(%r)
+assert F.fake_launches(b"kTileFill") == 1
+rows = live()
+assert F.fake_launches(b"kTileFill") == 1
+assert tiled - rows <= %d, tiled - rows
+""" % (without, held), tmp_path, SHCI_STORAGE=storage)
