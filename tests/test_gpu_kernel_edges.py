@@ -105,16 +105,16 @@ def test_screening_of_few_sources(case, n, eps, tmp_path):
     np.testing.assert_array_equal(got, want)
 
 
-@pytest.mark.parametrize("n", [3, 8, 257, 1500])
-@pytest.mark.parametrize("roots", [1, 2, 9])
+@pytest.mark.parametrize("n,roots", [(n, r) for n in (3, 8, 257, 1500) for r in (1, 2, 9) if r <= n])
 def test_davidson_subspaces(n, roots, tmp_path):
-    """Every subspace size, up to 12 columns and up to the whole space, and
-    vectors shorter than a workgroup: roots against the dense eigenvalues of
-    the GPU's own rows to 1e-8 (a residual below 1e-5, so the square of it
-    over the gaps)."""
+    """Subspaces that grow to 4, 5 and 12 columns or to the whole space, and
+    vectors shorter than a workgroup: from random vectors, orthonormal
+    eigenvectors of the GPU's own rows (residuals of the tolerance 1e-5; a root
+    found twice would overlap by 1) with eigenvalues of the dense matrix to 1e-8
+    (the square of the residual over the gaps); from the lowest eigenvectors with
+    noise, the lowest eigenvalues, each once (to 4e-8: residuals up to 2e-5, gaps
+    from 0.0128 on)."""
     from dice_amd import shci
-    if roots + 3 > 12 or roots > n:
-        pytest.skip("more roots than determinants")
     path, occ, W = _system("w1", tmp_path)
     dets = _space(path, occ, n, W)
     s = shci.System.from_fcidump(path)
@@ -124,16 +124,21 @@ def test_davidson_subspaces(n, roots, tmp_path):
     for i in range(n):
         H[i, cols[rp[i]:rp[i + 1]]] = vals[rp[i]:rp[i + 1]]
     H = np.tril(H) + np.tril(H, -1).T
-    x0 = np.random.default_rng(n).normal(size=(n, roots))
+    ev, U = np.linalg.eigh(H)
+    rng = np.random.default_rng(n)
+    x0 = rng.normal(size=(n, roots))
     x0[:roots] += 5.0 * np.eye(roots)
-    e, x, _ = s.davidson(x0, max_copies=max(roots + 3, 4), tol=1e-5)
-    resid = np.linalg.norm(H @ x - x * e, axis=0)
-    assert np.max(resid) < 2e-5
-    if n <= 8:
-        np.testing.assert_allclose(e, np.linalg.eigvalsh(H)[:roots], rtol=0, atol=1e-8)
-    else:
-        ev = np.linalg.eigvalsh(H)
-        assert all(np.min(np.abs(ev - v)) < 1e-8 for v in e)
+    noise = rng.normal(size=(n, roots)) * 0.02 / np.sqrt(n)
+    for start, low in ((x0, False), (U[:, :roots] + noise, True)):
+        e, x, _ = s.davidson(start, max_copies=max(roots + 3, 4), tol=1e-5)
+        assert np.max(np.linalg.norm(H @ x - x * e, axis=0)) < 2e-5
+        assert np.max(np.abs(x.T @ x - np.eye(roots))) < 1e-6
+        if low:
+            np.testing.assert_allclose(e, ev[:roots], rtol=0, atol=4e-8)
+        elif n <= 8:
+            np.testing.assert_allclose(e, ev[:roots], rtol=0, atol=1e-8)
+        else:
+            assert all(np.min(np.abs(ev - v)) < 1e-8 for v in e)
 
 
 @pytest.mark.parametrize("half", [True, False])
