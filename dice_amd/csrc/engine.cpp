@@ -1481,7 +1481,7 @@ std::vector<double> Engine::davidson(double* dX0, int nr, int maxCopies, double 
   };
   auto dotHost = [&](const double* a, const double* b) {
     double v;
-    launchGram(a, 1, b, 1, N, N, sc + 2, dvPart, s);
+    launchDot(a, b, N, sc + 2, dvPart, s);
     readScalars(&v, sc + 2, 1);
     return v;
   };

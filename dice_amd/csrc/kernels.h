@@ -337,9 +337,8 @@ void launchRayleighRitz(double* B, double* S, int m, int64_t n, double* w, doubl
 // columns one after the other, and normalised into dst
 void launchCorrection(double* r, const double* diag, const double* e, const double* B, int m, int64_t n, double* dst,
                       DevMem& partial, hipStream_t s);
-// G[0] = A . B (one column each)
-void launchGram(const double* A, int ma, const double* B, int mb, int64_t n, int64_t ld, double* G,
-                DevMem& partial, hipStream_t s);
+// *out = a . b
+void launchDot(const double* a, const double* b, int64_t n, double* out, DevMem& partial, hipStream_t s);
 // out[i*cols + j] = C[i*ldc + j] for i < rows, j < cols (small matrices)
 void launchSubMatrix(const double* C, int ldc, int rows, int cols, double* out, hipStream_t s);
 // G[i*mb + j] = A[:,i] . B[:,j] for ma, mb <= 64 (8 x 8 tiles; fixed-order sums);

@@ -123,14 +123,9 @@ __global__ void kCmax(const double* ci, int nroots, int64_t ld, int64_t n, doubl
 // emit one candidate per lane with `want`, skipping determinants already in
 // the variational space; wave-aggregated append
 template <int W>
-__device__ __forceinline__ void emitCandidate(bool want, const uint64_t* candIn, const int32_t* table, uint64_t mask,
+__device__ __forceinline__ void emitCandidate(bool want, const uint64_t* cand, const int32_t* table, uint64_t mask,
                                               const uint64_t* dets, uint64_t* out, unsigned long long* counter,
-                                              int64_t cap, bool trev = false) {
-  // with time reversal the space holds standard forms (SHCI/SHCIbasics.cpp:984-996)
-  uint64_t cand[W];
-#pragma unroll
-  for (int w = 0; w < W; w++) cand[w] = candIn[w];
-  if (trev) makeStandardForm<W>(cand);
+                                              int64_t cap) {
   bool keep = want && !hashContains<W>(table, mask, dets, cand);
   uint64_t m = __ballot(keep);
   if (m == 0) return;
@@ -178,6 +173,7 @@ struct CandidateQueue {
     uint64_t cand[W];
 #pragma unroll
     for (int w = 0; w < W; w++) cand[w] = candIn[w];
+    // with time reversal the space holds standard forms (SHCI/SHCIbasics.cpp:984-996)
     if (trev) makeStandardForm<W>(cand);
     const bool keep = want && !hashContains<W>(table, mask, dets, cand);
     const uint64_t m = __ballot(keep);
@@ -1238,7 +1234,6 @@ __global__ void kGroupStarts(const uint64_t* key, int64_t n, uint64_t nminor, in
   }
 }
 
-// alpha strings one excitation away from each unique alpha string
 // Bitmaps of the large alpha groups over the beta strings: per 64 strings a
 // word, and the members of the group before it.  flag: 1 for a group with
 // one; scanned, its slot.
@@ -1284,6 +1279,7 @@ __global__ void kBitmapCounts(const int64_t* slot, int64_t nA, int64_t words, in
   }
 }
 
+// alpha strings one excitation away from each unique alpha string
 template <bool FILL>
 __global__ void kStringSingles(const uint64_t* sorted, int64_t ns, int norb, const int64_t* start, int64_t* count,
                                uint32_t* out) {
@@ -2921,60 +2917,6 @@ constexpr int kRedBlocks = 512;
 // workgroups to keep every SIMD busy with latency-bound work
 constexpr int kPtRedBlocks = 8192;
 
-// per-block partial Gram entries, then a fixed-order final sum
-template <int MA, int MB>
-__global__ void __launch_bounds__(kBlock) kGramPartial(const double* A, const double* B, int ma, int mb, int64_t n,
-                                                       int64_t ld, double* partial) {
-  __shared__ double red[kWaves][MA * MB];
-  double acc[MA * MB];
-#pragma unroll
-  for (int q = 0; q < MA * MB; q++) acc[q] = 0.0;
-  for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x) {
-    double a[MA], bb[MB];
-#pragma unroll
-    for (int i = 0; i < MA; i++) a[i] = i < ma ? A[i * ld + k] : 0.0;
-#pragma unroll
-    for (int j = 0; j < MB; j++) bb[j] = j < mb ? B[j * ld + k] : 0.0;
-#pragma unroll
-    for (int i = 0; i < MA; i++)
-#pragma unroll
-      for (int j = 0; j < MB; j++) acc[i * MB + j] = fma(a[i], bb[j], acc[i * MB + j]);
-  }
-  const int wave = threadIdx.x >> 6, lane = __lane_id();
-#pragma unroll
-  for (int q = 0; q < MA * MB; q++) {
-    double v = acc[q];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    if (lane == 0) red[wave][q] = v;
-  }
-  __syncthreads();
-  for (int q = threadIdx.x; q < MA * MB; q += blockDim.x) {
-    double v = 0.0;
-    for (int w = 0; w < kWaves; w++) v += red[w][q];
-    partial[(int64_t)blockIdx.x * MA * MB + q] = v;
-  }
-}
-
-// one block per output: fixed-order strided partial sums, then a block tree
-__global__ void __launch_bounds__(kBlock) kGramFinal(const double* partial, int nblocks, int MA, int MB, int ma,
-                                                     int mb, double* G) {
-  __shared__ double red[kWaves];
-  const int q = blockIdx.x;
-  const int i = q / mb, j = q % mb;
-  double v = 0.0;
-  for (int b = threadIdx.x; b < nblocks; b += blockDim.x) v += partial[(int64_t)b * MA * MB + i * MB + j];
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  if (__lane_id() == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = 0.0;
-    for (int w = 0; w < kWaves; w++) t += red[w];
-    G[i * mb + j] = t;
-  }
-}
-
 __device__ __forceinline__ double shflXor(double v, int o) { return __shfl_xor(v, o, 64); }
 
 // acc[0 .. 2 O) over the wave: lanes with bit O keep the upper O sums.  Each
@@ -3332,6 +3274,14 @@ __global__ void kOrthoStep(double* r, const double* b, const double* d, int64_t 
     r[k] = r[k] - ov * b[k] / nn;
 }
 
+__global__ void __launch_bounds__(kBlock) kDot(const double* a, const double* b, int64_t n, double* partial) {
+  double s = 0.0;
+  for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x)
+    s = fma(a[k], b[k], s);
+  double t = blockSum(s);
+  if (threadIdx.x == 0) partial[blockIdx.x] = t;
+}
+
 __global__ void __launch_bounds__(kBlock) kNorm2(const double* x, int64_t n, double* partial) {
   double s = 0.0;
   for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x)
@@ -3440,7 +3390,7 @@ __device__ void jacobiWave(double* a, double* v, int* order, int m, double* w, d
 // and every sum takes the operations of separate kernels for the Gram matrix,
 // its eigenpairs, the rotation, the residual, the preconditioner, each dot
 // product, each orthogonalisation step and the norms, in their order: the
-// same bits.  With m columns m + 7 launches in place of 3 m + 13 and more, and
+// same bits.  With m columns m + 6 launches in place of 3 m + 12 and more, and
 // the scalars the host decides on come through memory it can read.  The
 // two-root solve on 57,963 determinants of 40 orbitals (184 iterations) 52 ->
 // 30 ms, the whole step of an 8-orbital molecule (86 iterations) 20 -> 16.
@@ -3530,7 +3480,7 @@ __global__ void __launch_bounds__(kBlock) kGramUpper(const double* __restrict__ 
 }
 
 // the Gram matrix from those partials (a wave per entry: the four wave sums
-// of kGramFinal one after the other) and its eigenpairs; one workgroup
+// of kFinalSum one after the other) and its eigenpairs; one workgroup
 constexpr int kGramThreads = 1024;
 __global__ void __launch_bounds__(kGramThreads) kGramJacobi(const double* __restrict__ partial, int nb, int m,
                                                             double* w, double* V) {
@@ -4854,17 +4804,11 @@ void launchSymRowBound(const TiledHam& T, const uint32_t* pos, const uint32_t* b
   HIP_CHECK(hipGetLastError());
 }
 
-void launchGram(const double* A, int ma, const double* B, int mb, int64_t n, int64_t ld, double* G, DevMem& partial,
-                hipStream_t s) {
-  const int nb = (int)std::min<int64_t>(kRedBlocks, (n + kBlock - 1) / kBlock);
-  const int nbb = nb < 1 ? 1 : nb;
-  if (ma <= 1 && mb <= 1) {
-    partial.reserve((size_t)nbb * 1 * sizeof(double));
-    kGramPartial<1, 1><<<nbb, kBlock, 0, s>>>(A, B, ma, mb, n, ld, partial.as<double>());
-    kGramFinal<<<ma * mb, kBlock, 0, s>>>(partial.as<double>(), nbb, 1, 1, ma, mb, G);
-  } else {
-    throw HipError("launchGram: subspace too large");
-  }
+void launchDot(const double* a, const double* b, int64_t n, double* out, DevMem& partial, hipStream_t s) {
+  const int nb = (int)std::max<int64_t>(1, std::min<int64_t>(kRedBlocks, (n + kBlock - 1) / kBlock));
+  partial.reserve((size_t)nb * sizeof(double));
+  kDot<<<nb, kBlock, 0, s>>>(a, b, n, partial.as<double>());
+  kFinalSum<<<1, kBlock, 0, s>>>(partial.as<double>(), nb, 1, 1, out);
   HIP_CHECK(hipGetLastError());
 }
 
