@@ -1435,8 +1435,9 @@ __device__ __forceinline__ int waveMaxScan(int v) {
 // groups of alpha strings one excitation away whose beta string is one
 // excitation away.  Group members are in increasing determinant index, so
 // jmin and jmax leave a prefix and a suffix of each group out (binary search).
-// Bound by VALU work (55% of the cycles): per 64 candidates finding their
-// groups, one popcount each, and the count or the queue.
+// Bound by the vector memory path (TD 95% busy, the L1 waiting for misses 61%
+// of the time, VALU 44 and 52% busy in the count and the fill pass): each
+// group member's string, the bitmap words, and the elements' integrals.
 template <class Sink>
 __device__ __forceinline__ void enumerateRow(const RowTables& T, int64_t I, uint32_t jmin, uint32_t jmax,
                                              int wave, int lane,
@@ -2504,19 +2505,23 @@ __global__ void __launch_bounds__(kBlock) kSigmaTiled(const uint2* __restrict__ 
 //
 // How the work is cut changes no bit, so the instructions are taken in an
 // order of their own: kSymBlocks row blocks form a super block, whose
-// instructions are sorted by tile (SymOrder).  A workgroup then keeps the x
+// instructions are sorted by tile (buildSymOrder).  A workgroup then keeps the x
 // and the sums of the super block's rows and of the current tile's columns
 // in LDS (32 KB, four workgroups of 512 threads per CU) for all the entries
 // of that tile, so that nothing but the entries is read from memory per
-// entry, and a tile's sums are added to yT once for 1,024 rows.  Bound by the
-// scan's VALU work and the LDS adds beside HBM.
+// entry, and a tile's sums are added to yT once for 1,024 rows.  Bound by what
+// it does per entry (VALU 59% busy, the LDS adds, the wait for the entries),
+// not by bytes: with FP32 values it moves 8.6 GB a launch for 11.6 and takes as
+// long.
 //
-// Measured, one product, against a workgroup per row block whose four waves
+// Measured, one product and the wait for it, against a workgroup per row block whose four waves
 // each kept a tile's transposed sums of their own and gathered x through L1:
 // 2,471 determinants of 16 orbitals 61 -> 15 us, 27,685 of 24 orbitals 423 ->
 // 55, 57,963 of 40 orbitals 371 -> 89, 200,003 of 24 orbitals 569 -> 239,
 // 1,000,003 of them (4.7e8 pairs) 2,569 -> 1,700 (3.3 TB/s over 12 bytes a
-// pair), 300,007 of 40 orbitals with FP32 values 1,930 -> 980.  Super blocks
+// pair), 300,007 of 40 orbitals with FP32 values 1,930 -> 980.  One after the
+// other without a wait, where the old split's launches overlapped, the million
+// 2,241 -> 1,598, two FP32 vectors of the 300,007 1,951 -> 1,702.  Super blocks
 // of 2 and 8 blocks: 2,000 and 1,700 us on the million, 97 and 90 on the
 // 57,963; 256 threads: 1,990 and 109; 2 and 8 instructions at a time: 1,730
 // and 1,800.
@@ -3107,7 +3112,8 @@ inline size_t ptTabBytes(int n) { return ((size_t)n + 2 * (size_t)n * n) * sizeo
 template <int W, bool LDS_TAB>
 __device__ __forceinline__ double ptEnergy(const DevSystem& S, const double* tab, const uint64_t* d) {
   // (the same additions in the same order as Energy(): E_a is bit-identical,
-  // which matters for external determinants whose E0 - E_a is small)
+  // which matters for external determinants whose E0 - E_a is small; for the
+  // others a sum from the source's energy would do)
   if (LDS_TAB) return detEnergyTab<W>(tab, tab + S.norb, tab + S.norb + S.norb * S.norb, S.norb, d);
   return detEnergy<W>(S, d);
 }
